@@ -47,7 +47,33 @@ __device__ __forceinline__ const NF_CONST T *cptr(const void *p) {
     return (const NF_CONST T *)(p);
 }
 
-__device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
+// Transcendentals at raised wave priority.  gfx950 issues plain FP32 VALU
+// instructions of two waves of a SIMD together (16 v_mul_f32 of VGPRs take 37
+// cycles with 8 waves, 2.3 each; 4.3 each when every one reads an SGPR), but
+// after a v_rsq_f32 that the arbiter interleaves with other waves the SIMD
+// falls back to one instruction per 4 cycles: v_rsq + 11 v_mul take 53 cycles.
+// s_setprio around it keeps the pairing: a pair of 11 VALU instructions and a
+// v_rsq takes 34-37 cycles instead of 41-54.  The s_setprio after it is also
+// the wait state that a VALU use of a transcendental's result needs.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define NF_TRANS1(op, a) asm("s_setprio 3\n\t" op " %0, %0\n\ts_setprio 0" : "+v"(a))
+#define NF_TRANS2(op, a, b) asm("s_setprio 3\n\t" op " %0, %0\n\t" op " %1, %1\n\ts_setprio 0" : "+v"(a), "+v"(b))
+#else
+#define NF_TRANS1(op, a) (void)(a)
+#define NF_TRANS2(op, a, b) (void)(a), (void)(b)
+#endif
+__device__ __forceinline__ float rsq(float x) {
+    NF_TRANS1("v_rsq_f32", x);
+    return x;
+}
+__device__ __forceinline__ float sqrt_(float x) {
+    NF_TRANS1("v_sqrt_f32", x);
+    return x;
+}
+__device__ __forceinline__ float rcp(float x) {
+    NF_TRANS1("v_rcp_f32", x);
+    return x;
+}
 __device__ __forceinline__ float clamp01(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); }
 
 // A SIC's counts: from device memory when it was planned on the device
@@ -491,7 +517,7 @@ __device__ __forceinline__ void ref_pair(float sx, float sy, float sz, float kx,
         f = r * r * r;
     } else if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE) {
         const float rinv = rsq(r2);
-        const float u = pc.eps * __builtin_amdgcn_sqrtf(r2);  // eps_inv / rinv
+        const float u = pc.eps * sqrt_(r2);  // eps_inv / rinv
         if (u >= 2.0f) {
             f = rinv * rinv * rinv;
         } else if (u >= 1.0f) {
@@ -506,7 +532,7 @@ __device__ __forceinline__ void ref_pair(float sx, float sy, float sz, float kx,
         float r = r2 + 1e-16f;
         r *= r * rsq(r);
         r += pc.eps;
-        f = __builtin_amdgcn_rcpf(r);
+        f = rcp(r);
     }
     ax -= f * dx;
     ay -= f * dy;
@@ -677,44 +703,100 @@ __global__ __launch_bounds__(256) void k_coadd_f64_group(const GroupSic *__restr
 // The unsoftened branch equals the full form for every pair with r > e.
 constexpr int kNoDensity = 0, kDensity = 1, kExact = 2;
 
-template <int SOFT, int MODE>
-__device__ __forceinline__ void pair_box(float sx, float sy, float sz, float kx, float ky, float kz,
-                                         const PairConst &pc, float &ax, float &ay, float &az, float &aw) {
-    const float dx = sx - kx, dy = sy - ky, dz = sz - kz;
-    float r2 = fmaf(dx, dx, pc.r2add);
+// A pair in four steps, so that the transcendentals of two pairs can run in
+// one raised stretch (35.9 -> 35.4 cycles per pair):
+// 1. d = sink - source (so that a += g d, and no operand of an FMA carries a
+//    sign), r2 and the density term;
+template <int MODE>
+__device__ __forceinline__ void pair_r2(float sx, float sy, float sz, float kx, float ky, float kz,
+                                        const PairConst &pc, float &dx, float &dy, float &dz, float &r2, float &aw) {
+    dx = kx - sx;
+    dy = ky - sy;
+    dz = kz - sz;
+    r2 = fmaf(dx, dx, pc.r2add);
     r2 = fmaf(dy, dy, r2);
     r2 = fmaf(dz, dz, r2);
     if constexpr (MODE != kNoDensity) aw += clamp01(pc.b2x - r2);
-    float g;
-    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE) {
-        const float f = rsq(r2);
-        const float f3 = f * f * f;
-        if constexpr (MODE != kExact) g = f3;
-        else g = fminf(f3, fmaf(fmaf(pc.c1, f, pc.c2), r2, pc.c3));
-    } else if constexpr (SOFT == NF_SOFT_PLUMMER) {
-        const float f = rsq(r2);
-        g = f * f * f;
-    } else if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE) {
-        const float rinv = rsq(r2);
-        const float u = pc.eps * __builtin_amdgcn_sqrtf(r2);
-        if (u >= 2.0f) {
-            g = rinv * rinv * rinv;
-        } else if (u >= 1.0f) {
-            const float u3 = u * u * u;
-            g = rinv * rinv * rinv *
-                ((float)(-1.0 / 15.0) + (float)(8.0 / 3.0) * u3 - 3.0f * u3 * u + (float)(6.0 / 5.0) * u3 * u * u -
-                 (float)(1.0 / 6.0) * u3 * u3);
-        } else {
-            g = pc.eps * pc.eps * pc.eps * ((float)(4.0 / 3.0) - (float)(6.0 / 5.0) * u * u + 0.5f * u * u * u);
-        }
-    } else {  // cubic Plummer; r2 already holds + TAU2.  r^3 as r2*sqrt(r2) so a
-              // padding source (r2 = inf) gives 1/inf = 0, not inf*0.
-        const float r = r2 * __builtin_amdgcn_sqrtf(r2) + pc.eps;
-        g = __builtin_amdgcn_rcpf(r);
+}
+// 2. f = 1/r, or r for the cubic Plummer form;
+template <int SOFT>
+__device__ __forceinline__ void pair_f(float &a) {
+    if constexpr (SOFT == NF_SOFT_CUBIC_PLUMMER) NF_TRANS1("v_sqrt_f32", a);
+    else NF_TRANS1("v_rsq_f32", a);
+}
+template <int SOFT>
+__device__ __forceinline__ void pair_f(float &a, float &b) {
+    if constexpr (SOFT == NF_SOFT_CUBIC_PLUMMER) NF_TRANS2("v_sqrt_f32", a, b);
+    else NF_TRANS2("v_rsq_f32", a, b);
+}
+// 3. g from r2 and f;
+template <int SOFT, int MODE>
+__device__ __forceinline__ float pair_g(float r2, float f, const PairConst &pc) {
+    if constexpr (SOFT == NF_SOFT_CUBIC_PLUMMER) {
+        // r2 already holds + TAU2.  r^3 as r2*sqrt(r2), so a padding source
+        // (r2 = inf) gives 1/inf = 0, not inf*0.
+        return rcp(fmaf(r2, f, pc.eps));
     }
-    ax = fmaf(-g, dx, ax);
-    ay = fmaf(-g, dy, ay);
-    az = fmaf(-g, dz, az);
+    const float f3 = f * f * f;
+    if constexpr (MODE != kExact || SOFT == NF_SOFT_PLUMMER) {
+        return f3;
+    } else if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE) {
+        return fminf(f3, fmaf(fmaf(pc.c1, f, pc.c2), r2, pc.c3));
+    } else {
+        // Cubic spline, u = r/e: f^3 beyond 2, below it e^-3 times a cubic in u
+        // (from 1 on, with the -1/(15 u^3) of the middle piece as -f^3/15).
+        // Selects, not branches: nearly every wave has lanes in each piece.  A
+        // padding source (r2 = inf, f = 0) has u = NaN and takes f^3 = 0.
+        const float u = r2 * f * pc.eps;
+        const float mid = fmaf(fmaf(fmaf((float)(-1.0 / 6.0), u, (float)(6.0 / 5.0)), u, -3.0f), u, (float)(8.0 / 3.0));
+        const float in = fmaf(fmaf(0.5f, u, (float)(-6.0 / 5.0)), u * u, (float)(4.0 / 3.0));
+        const bool outer = u >= 1.0f;
+        const float soft = fmaf(outer ? mid : in, pc.c3, outer ? f3 * (float)(-1.0 / 15.0) : 0.0f);
+        return u < 2.0f ? soft : f3;
+    }
+}
+// 4. the force sums.
+__device__ __forceinline__ void pair_sum(float g, float dx, float dy, float dz, float &ax, float &ay, float &az) {
+    ax = fmaf(g, dx, ax);
+    ay = fmaf(g, dy, ay);
+    az = fmaf(g, dz, az);
+}
+
+template <int SOFT, int MODE>
+__device__ __forceinline__ void pair_box(float sx, float sy, float sz, float kx, float ky, float kz,
+                                         const PairConst &pc, float &ax, float &ay, float &az, float &aw) {
+    float dx, dy, dz, r2;
+    pair_r2<MODE>(sx, sy, sz, kx, ky, kz, pc, dx, dy, dz, r2, aw);
+    float f = r2;
+    pair_f<SOFT>(f);
+    pair_sum(pair_g<SOFT, MODE>(r2, f, pc), dx, dy, dz, ax, ay, az);
+}
+
+// The pairs of P sources (at sp) with the S sinks of a lane, sink slots below
+// S/2 in form MLO and the others in MHI.
+template <int SOFT, int MLO, int MHI, int S, int P>
+__device__ __forceinline__ void pair_group(const NF_CONST float4 *sp, const float *kx, const float *ky,
+                                           const float *kz, const PairConst &pc, float *bx, float *by, float *bz,
+                                           float *tw) {
+    constexpr int N = P * S;
+    float dx[N], dy[N], dz[N], r2[N], f[N];
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+        const int u = t % S;
+        const float4 sv = sp[t / S];
+        if (u < S / 2) pair_r2<MLO>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, dx[t], dy[t], dz[t], r2[t], tw[u]);
+        else pair_r2<MHI>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, dx[t], dy[t], dz[t], r2[t], tw[u]);
+        f[t] = r2[t];
+    }
+    if constexpr (N == 1) pair_f<SOFT>(f[0]);
+#pragma unroll
+    for (int t = 0; t + 1 < N; t += 2) pair_f<SOFT>(f[t], f[t + 1]);
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+        const int u = t % S;
+        const float g = u < S / 2 ? pair_g<SOFT, MLO>(r2[t], f[t], pc) : pair_g<SOFT, MHI>(r2[t], f[t], pc);
+        pair_sum(g, dx[t], dy[t], dz[t], bx[u], by[u], bz[u]);
+    }
 }
 
 // TwoSum (Knuth): s + e == a + b exactly.
@@ -784,8 +866,7 @@ __device__ __forceinline__ float3 pencil_sink(const SicView &v, const SinkCells 
 // and the sinks' bounding box (wave-uniform).
 template <int SOFT>
 __device__ __forceinline__ int tile_mode(const BatchCtx &cx, float gap2) {
-    if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE || SOFT == NF_SOFT_CUBIC_PLUMMER) return kExact;
-    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE)
+    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE || SOFT == NF_SOFT_CUBIC_SPLINE)
         if (!cx.pc.fast_ok || gap2 <= cx.soft2) return kExact;
     return gap2 <= cx.dens2 ? kDensity : kNoDensity;
 }
@@ -822,21 +903,15 @@ template <int SOFT, int MLO, int MHI, int S>
 __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, const float *kx, const float *ky,
                                           const float *kz, const PairConst &pc, float *tx, float *ty, float *tz,
                                           float *tw) {
+    constexpr int P = S == 1 ? 2 : 1;  // sources per pair_group
     const int fullb = cnt & ~(kSrcBatch - 1);
     for (int i = 0; i < fullb; i += kSrcBatch) {
         float bx[S], by[S], bz[S];
 #pragma unroll
         for (int u = 0; u < S; u++) bx[u] = by[u] = bz[u] = 0.f;
 #pragma unroll
-        for (int q = 0; q < kSrcBatch; q++) {
-            const float4 sv = sp[i + q];
-#pragma unroll
-            for (int u = 0; u < S / 2; u++)
-                pair_box<SOFT, MLO>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, bx[u], by[u], bz[u], tw[u]);
-#pragma unroll
-            for (int u = S / 2; u < S; u++)
-                pair_box<SOFT, MHI>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, bx[u], by[u], bz[u], tw[u]);
-        }
+        for (int q = 0; q < kSrcBatch; q += P)
+            pair_group<SOFT, MLO, MHI, S, P>(sp + i + q, kx, ky, kz, pc, bx, by, bz, tw);
 #pragma unroll
         for (int u = 0; u < S; u++) {
             tx[u] += bx[u];
@@ -848,15 +923,7 @@ __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, co
         float bx[S], by[S], bz[S];
 #pragma unroll
         for (int u = 0; u < S; u++) bx[u] = by[u] = bz[u] = 0.f;
-        for (int q = fullb; q < cnt; q++) {
-            const float4 sv = sp[q];
-#pragma unroll
-            for (int u = 0; u < S / 2; u++)
-                pair_box<SOFT, MLO>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, bx[u], by[u], bz[u], tw[u]);
-#pragma unroll
-            for (int u = S / 2; u < S; u++)
-                pair_box<SOFT, MHI>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, bx[u], by[u], bz[u], tw[u]);
-        }
+        for (int q = fullb; q < cnt; q++) pair_group<SOFT, MLO, MHI, S, 1>(sp + q, kx, ky, kz, pc, bx, by, bz, tw);
 #pragma unroll
         for (int u = 0; u < S; u++) {
             tx[u] += bx[u];
@@ -1499,9 +1566,12 @@ int launch_batched(const SicView *views, int cpd, int softening, const PairConst
     BatchCtx cx;
     cx.pc = pc;
     cx.invcpd = 1.0 / (double)cpd;
-    // The unsoftened branch is exact for r^2 > e^2 = 1/eps; the box test uses
-    // a relative margin far above FP32 rounding of the box corners.
-    cx.soft2 = (softening == NF_SOFT_SINGLE_SPLINE) ? (float)((1.0 / (double)pc.eps) * 1.01) : 0.f;
+    // The unsoftened branch is exact for r^2 > e^2 = 1/eps (single spline) and
+    // for r > 2 e = 2/eps (cubic spline); the box test uses a relative margin
+    // far above FP32 rounding of the box corners.
+    cx.soft2 = softening == NF_SOFT_SINGLE_SPLINE  ? (float)((1.0 / (double)pc.eps) * 1.01)
+               : softening == NF_SOFT_CUBIC_SPLINE ? (float)(4.0 / ((double)pc.eps * (double)pc.eps) * 1.01)
+                                                   : 0.f;
     // Density is nonzero only for r^2 + r2add < b2x; a 1% margin covers the
     // FP32 rounding of the box gap and of r^2.
     cx.dens2 = pc.b2x > 0.f ? (float)((double)pc.b2x * 1.01) : -1.f;

@@ -126,7 +126,7 @@ struct PairConst {
     float b2;         // FOF density radius^2 as given
     float r2add;      // added to r^2 before rsqrt: tau (spline forms) or e^2 (Plummer)
     float b2x;        // density threshold against that r^2: b2 + r2add
-    float c1, c2, c3; // single spline, box-unit polynomial (-15 e^-4, 6 e^-5, 10 e^-3)
+    float c1, c2, c3; // single spline, box-unit polynomial (-15 e^-4, 6 e^-5, 10 e^-3); cubic spline: c3 = e^-3
     float theta;      // tile density sum below which no pair is softened (< 0: none)
     double out_scale; // e^3 for the box-unit spline, 1 otherwise
     int32_t fast_ok;  // 1 when the unsoftened fast path may be used

@@ -71,7 +71,11 @@ int derive_pair_const(int softening, float eps, float b2, PairConst *pc) {
             break;
         }
         case NF_SOFT_PLUMMER: pc->r2add = eps; break;
-        case NF_SOFT_CUBIC_SPLINE: pc->r2add = 0.f; break;
+        case NF_SOFT_CUBIC_SPLINE:
+            pc->r2add = 1e-24f;  // as the single spline's: keeps the self pair's 1/r finite
+            pc->c3 = eps * eps * eps;
+            pc->fast_ok = 1;
+            break;
         case NF_SOFT_CUBIC_PLUMMER: pc->r2add = 1e-16f; break;  // TAU2, DirectGPUKernels.cuh:113
         default: return fail(NF_ERR_INVALID, "unknown softening");
     }
