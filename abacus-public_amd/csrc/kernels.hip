@@ -799,28 +799,6 @@ __device__ __forceinline__ void pair_group(const NF_CONST float4 *sp, const floa
     }
 }
 
-// TwoSum (Knuth): s + e == a + b exactly.
-__device__ __forceinline__ void two_sum(float a, float b, float &s, float &e) {
-    s = a + b;
-    const float bb = s - a;
-    e = (a - (s - bb)) + (b - bb);
-}
-__device__ __forceinline__ void merge(float &h, float &l, float t) {
-    float s, e;
-    two_sum(h, t, s, e);
-    h = s;
-    l += e;
-}
-
-// Squared gap between two axis-aligned boxes (0 if they overlap).
-__device__ __forceinline__ float box_gap2(float alx, float aly, float alz, float ahx, float ahy, float ahz, float4 bl,
-                                          float4 bh) {
-    const float gx = fmaxf(0.f, fmaxf(bl.x - ahx, alx - bh.x));
-    const float gy = fmaxf(0.f, fmaxf(bl.y - ahy, aly - bh.y));
-    const float gz = fmaxf(0.f, fmaxf(bl.z - ahz, alz - bh.z));
-    return gx * gx + gy * gy + gz * gz;
-}
-
 struct BatchCtx {
     PairConst pc;
     double invcpd;
@@ -871,6 +849,66 @@ __device__ __forceinline__ int tile_mode(const BatchCtx &cx, float gap2) {
     return gap2 <= cx.dens2 ? kDensity : kNoDensity;
 }
 
+// A sink pencil's W source pencils: lane y holds pencil y's first slot and
+// count, pre[y] the 64-source blocks before pencil y (wave-uniform).  The
+// lookups of all W pencils are in flight together: a chain of two loads per
+// item, not per pencil.
+struct SourceRows {
+    int start, count;            // per lane
+    int pre[NF_MAX_WIDTH + 1];
+    __device__ __forceinline__ int start_of(int y) const { return __builtin_amdgcn_readlane(start, y); }
+    __device__ __forceinline__ int count_of(int y) const { return __builtin_amdgcn_readlane(count, y); }
+};
+__device__ __forceinline__ SourceRows source_rows(const SicView &v, int s, int lane) {
+    SourceRows r;
+    r.start = r.count = 0;
+    if (lane < v.W) {
+        const int si = cptr<int32_t>(v.ilist)[s * v.W + lane];
+        r.start = cptr<int32_t>(v.src_set_start)[si];
+        r.count = cptr<int32_t>(v.src_set_count)[si];
+    }
+    r.pre[0] = 0;
+#pragma unroll
+    for (int y = 0; y < NF_MAX_WIDTH; y++) r.pre[y + 1] = r.pre[y] + (r.count_of(y) + kWave - 1) / kWave;
+    return r;
+}
+// The pair forms of blocks p, p + 1, ... p + 63 of the pencils' blocks taken
+// one after the other, one per lane: form_lo | form_hi << 2 against the sinks'
+// boxes (x and y: bl, bh; z per half of the sink slots).
+struct SinkBox {
+    float lx, ly, hx, hy, lz0, hz0, lz1, hz1;
+};
+template <int SOFT, bool HALVES>
+__device__ __forceinline__ int block_forms(const BatchCtx &cx, const SicView &v, const SourceRows &r,
+                                           const SinkBox &k, int p, int lane) {
+    const NF_CONST float4 *box = cptr<float4>(v.box4);
+    const int i = p + lane;
+    int y = 0, first = 0;
+#pragma unroll
+    for (int c = 1; c < NF_MAX_WIDTH; c++) {
+        const bool in = i >= r.pre[c];
+        y = in ? c : y;
+        first = in ? r.pre[c] : first;
+    }
+    const int start = __shfl(r.start, y);
+    if (i >= r.pre[NF_MAX_WIDTH]) return 0;
+    const int64_t gb = (int64_t)start / kWave + (i - first);
+    const float4 ql = box[2 * gb], qh = box[2 * gb + 1];
+    const double yo = (double)(y - v.R) * cx.invcpd;
+    const float sly = (float)((double)k.ly - yo), shy = (float)((double)k.hy - yo);
+    const float gx = fmaxf(0.f, fmaxf(ql.x - k.hx, k.lx - qh.x));
+    const float gy = fmaxf(0.f, fmaxf(ql.y - shy, sly - qh.y));
+    const float gxy = gx * gx + gy * gy;
+    const float gz1 = fmaxf(0.f, fmaxf(ql.z - k.hz1, k.lz1 - qh.z));
+    const int mh = tile_mode<SOFT>(cx, gxy + gz1 * gz1);
+    int ml = mh;
+    if (HALVES) {
+        const float gz0 = fmaxf(0.f, fmaxf(ql.z - k.hz0, k.lz0 - qh.z));
+        ml = tile_mode<SOFT>(cx, gxy + gz0 * gz0);
+    }
+    return ml | (mh << 2);
+}
+
 // Pair interactions a wave has computed in each pair form (kNoDensity,
 // kDensity, kExact) and in short tails: wave-uniform, so the counts live in
 // scalar registers and cost no VALU work.  Counted only by the census
@@ -895,9 +933,9 @@ __device__ __forceinline__ void census_add(Census &c, int mode, uint64_t n) {
 // batch sums of 8 terms, which cost 1% more kernel time.  Sink slots
 // u < S/2 take pair form MLO, the others MHI (S = 1: MHI); every form gives
 // the same value for the pairs its box test admits, so the split changes
-// which code runs, not the result.  The last batch takes only the
-// cnt % kSrcBatch real sources: the padding sources after them give exact
-// zeros, so leaving them out changes no sum.
+// which code runs, not the result.  The last batch stops at the first multiple
+// of 4 past the cnt % kSrcBatch real sources: the padding sources give exact
+// zeros, so how many of them are taken changes no sum.
 constexpr int kSrcBatch = 16;
 template <int SOFT, int MLO, int MHI, int S>
 __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, const float *kx, const float *ky,
@@ -923,7 +961,11 @@ __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, co
         float bx[S], by[S], bz[S];
 #pragma unroll
         for (int u = 0; u < S; u++) bx[u] = by[u] = bz[u] = 0.f;
-        for (int q = fullb; q < cnt; q++) pair_group<SOFT, MLO, MHI, S, 1>(sp + q, kx, ky, kz, pc, bx, by, bz, tw);
+        // (by 4, the last of them padding: one wait for scalar loads per 4 sources)
+        for (int q = fullb; q < cnt; q += 4)
+#pragma unroll
+            for (int k = 0; k < 4; k += P)
+                pair_group<SOFT, MLO, MHI, S, P>(sp + q + k, kx, ky, kz, pc, bx, by, bz, tw);
 #pragma unroll
         for (int u = 0; u < S; u++) {
             tx[u] += bx[u];
@@ -960,14 +1002,10 @@ template <int SOFT, int S, bool CENSUS>
 __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int lane,
                                           Census &cen) {
     const NF_CONST float4 *src = cptr<float4>(v.sources4);
-    const NF_CONST float4 *box = cptr<float4>(v.box4);
-    const NF_CONST int32_t *sink_set_start = cptr<int32_t>(v.sink_set_start);
-    const NF_CONST int32_t *src_set_start = cptr<int32_t>(v.src_set_start);
-    const NF_CONST int32_t *src_set_count = cptr<int32_t>(v.src_set_count);
-    const NF_CONST int32_t *ilist = cptr<int32_t>(v.ilist);
     NF_GLOBAL double *out = (NF_GLOBAL double *)v.partial;
     const int s = w.sinkset;
-    const int base = sink_set_start[s] + w.first;
+    const int base = cptr<int32_t>(v.sink_set_start)[s] + w.first;
+    const SourceRows rows = source_rows(v, s, lane);
     const int nsink = w.nsink;  // 64*S, or fewer for a masked tail tile
     const uint64_t n_lo = (uint64_t)min(nsink, kWave * (S / 2)), n_hi = (uint64_t)nsink - n_lo;  // sinks per half
     const SinkCells sc = sink_cells(v, s);
@@ -1017,44 +1055,24 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
 #pragma unroll
     for (int u = 0; u < S; u++) hx[u] = hy[u] = hz[u] = hw[u] = 0.0;
 
+    const SinkBox kbox = {blx, bly, bhx, bhy, blz0, bhz0, blz1, bhz1};
     const int W = v.W;
+    int modes = 0, p = 0;  // p: blocks done; lane i: forms of block (p & ~63) + i
     for (int y = 0; y < W; y++) {
-        const int si = ilist[s * W + y];
-        const int st = src_set_start[si];
-        const int n = src_set_count[si];
+        const int st = rows.start_of(y), n = rows.count_of(y);
         // Source y + (y-R)/cpd == sink y - (y-R)/cpd on the other side; the
         // cell-centre offset is formed in FP64.
         const double yo = (double)(y - v.R) * cx.invcpd;
         float kyy[S];
 #pragma unroll
         for (int u = 0; u < S; u++) kyy[u] = (float)((double)ky[u] - yo);
-        const float sly = (float)((double)bly - yo), shy = (float)((double)bhy - yo);
         const int nblk = (n + kWave - 1) / kWave;
-        // Lane b decides the pair forms of block b of this source pencil (64
-        // blocks per pass): one vector pass instead of a wave-uniform box test
-        // and a dependent box load per block.
-        int modes = 0;  // lane i: mlo | mhi << 2 of block b + i, for the pass starting at block b
-        for (int b = 0; b < nblk; b++) {
-            if ((b & (kWave - 1)) == 0) {
-                const int bl = b + lane;
-                modes = 0;
-                if (bl < nblk) {
-                    const int64_t gb = (int64_t)st / kWave + bl;
-                    const float4 ql = box[2 * gb], qh = box[2 * gb + 1];
-                    const float gx = fmaxf(0.f, fmaxf(ql.x - bhx, blx - qh.x));
-                    const float gy = fmaxf(0.f, fmaxf(ql.y - shy, sly - qh.y));
-                    const float gxy = gx * gx + gy * gy;
-                    const float gz1 = fmaxf(0.f, fmaxf(ql.z - bhz1, blz1 - qh.z));
-                    const int mh = tile_mode<SOFT>(cx, gxy + gz1 * gz1);
-                    int ml = mh;
-                    if (S > 1) {
-                        const float gz0 = fmaxf(0.f, fmaxf(ql.z - bhz0, blz0 - qh.z));
-                        ml = tile_mode<SOFT>(cx, gxy + gz0 * gz0);
-                    }
-                    modes = ml | (mh << 2);
-                }
-            }
-            const int pm = __builtin_amdgcn_readlane(modes, b & (kWave - 1));
+        for (int b = 0; b < nblk; b++, p++) {
+            // Lane i decides the pair forms of block i of the item's source
+            // blocks (64 per pass): one vector pass instead of a wave-uniform
+            // box test and a dependent box load per block.
+            if ((p & (kWave - 1)) == 0) modes = block_forms<SOFT, (S > 1)>(cx, v, rows, kbox, p, lane);
+            const int pm = __builtin_amdgcn_readlane(modes, p & (kWave - 1));
             const int mlo = pm & 3, mhi = pm >> 2;
             const NF_CONST float4 *sp = src + st + b * kWave;
             const int cnt = min(kWave, n - b * kWave);
@@ -1086,169 +1104,152 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
     }
 }
 
-// Short tail of a pencil (fewer than kTailLanes sinks): the wave is four
-// groups of 16 lanes; each group takes SU sinks of the pass (4*SU sinks per
-// pass) and its lanes stride over the sources 16 apart.  Per-lane partial
-// sums are TwoSum-reduced within each group by a 4-level butterfly, which
-// reduces the four groups' sinks at once.
-constexpr int kGroupLanes = 16;
-constexpr int kGroups = kWave / kGroupLanes;
-
-// TwoSum butterfly within aligned groups of kGroupLanes lanes.
-__device__ __forceinline__ void group_two_sum(float &h, float &l) {
-    for (int off = kGroupLanes / 2; off >= 1; off >>= 1) {
-        const float h2 = __shfl_xor(h, off);
-        const float l2 = __shfl_xor(l, off);
-        float s, e;
-        two_sum(h, h2, s, e);
-        h = s;
-        l = l + l2 + e;
+// Short tail of a pencil (r < kTailLanes sinks): the sinks sit two to a lane
+// on L = ceil(r / 2) lanes, the wave holds G = 64 / L such groups, and group g
+// takes every G-th source of a block, from source g on.  One pass over the
+// sources whatever r is, all lanes busy but 64 - L G and one slot of an odd r.
+// The sources come through vector loads (one 16 B load per two pairs of a
+// lane, the same address on a group's lanes).  Each block's FP32 sums join
+// FP64 sums per lane, as a register tile's do, and a tree over the groups adds
+// those.
+//
+// Against the sources on 16-lane groups with up to 8 sinks per pass, which this
+// replaces: the direct kernel of 24 sparse slabs (129^2 pencils of 25 sinks
+// each) 3.30 -> 1.27 ms, of eight 512^3 slabs 14.77 -> 14.08 ms (the tails
+// alone took 1.25 ms of that).  Two loads in flight (kAhead) instead of four
+// measured 0.5% faster but on the sparse slabs.
+template <int SOFT, int MODE>
+__device__ __forceinline__ void tail_block(const float4 *bp, int cnt, int G, int full, int grp, const float *kx,
+                                           const float *ky, const float *kz, const PairConst &pc, float *tx,
+                                           float *ty, float *tz, float *tw) {
+    auto pairs = [&](float4 sv) {
+        float dx[2], dy[2], dz[2], r2[2], f[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            pair_r2<MODE>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, dx[u], dy[u], dz[u], r2[u], tw[u]);
+            f[u] = r2[u];
+        }
+        pair_f<SOFT>(f[0], f[1]);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            pair_sum(pair_g<SOFT, MODE>(r2[u], f[u], pc), dx[u], dy[u], dz[u], tx[u], ty[u], tz[u]);
+    };
+    constexpr int kAhead = 2;  // loads in flight
+    int i = 0;
+    for (; i + kAhead <= full; i += kAhead) {
+        float4 sv[kAhead];
+#pragma unroll
+        for (int q = 0; q < kAhead; q++) sv[q] = bp[(i + q) * G + grp];
+#pragma unroll
+        for (int q = 0; q < kAhead; q++) pairs(sv[q]);
+    }
+    if (i * G < cnt) {  // the last steps: a group past the block's sources takes a padding source
+        float4 sv[kAhead];
+#pragma unroll
+        for (int q = 0; q < kAhead; q++) sv[q] = bp[min((i + q) * G + grp, cnt - 1)];
+#pragma unroll
+        for (int q = 0; q < kAhead; q++) {
+            if ((i + q) * G >= cnt) break;
+            if ((i + q) * G + grp >= cnt) sv[q].x = kFar;
+            pairs(sv[q]);
+        }
     }
 }
-__device__ __forceinline__ double group_sum(double v) {
-    for (int off = kGroupLanes / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
 
-template <int SOFT, int SU, bool CENSUS>
-__device__ __forceinline__ void rem_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int lane,
-                                         Census &cen) {
-    constexpr int TC = 16;  // 64-source blocks per TwoSum tile
-    const NF_CONST float4 *box = cptr<float4>(v.box4);
-    const NF_CONST int32_t *sink_set_start = cptr<int32_t>(v.sink_set_start);
-    const NF_CONST int32_t *src_set_start = cptr<int32_t>(v.src_set_start);
-    const NF_CONST int32_t *src_set_count = cptr<int32_t>(v.src_set_count);
-    const NF_CONST int32_t *ilist = cptr<int32_t>(v.ilist);
+template <int SOFT, bool CENSUS>
+__device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int lane,
+                                          Census &cen) {
     const float4 *src = static_cast<const float4 *>(v.sources4);
     NF_GLOBAL double *out = (NF_GLOBAL double *)v.partial;
     const int s = w.sinkset;
-    const int base = sink_set_start[s] + w.first;
+    const int base = cptr<int32_t>(v.sink_set_start)[s] + w.first;
+    const SourceRows rows = source_rows(v, s, lane);
     const int r = w.nsink;
-    const int W = v.W;
-    const int grp = lane / kGroupLanes, gl = lane % kGroupLanes;
+    const int L = (r + 1) / 2, G = kWave / L;
+    const int g = lane / L, slot = lane - g * L;
+    const int grp = min(g, G - 1);  // (lanes past the last group repeat it, and join no sum)
     const SinkCells sc = sink_cells(v, s);
-    for (int g0 = 0; g0 < r; g0 += kGroups * SU) {
-        // This group's sinks: g0 + grp*SU + u (repeats of the last sink past
-        // the tail are computed and not stored).
-        float kx[SU], ky[SU], kz[SU];
-        float blx = __builtin_huge_valf(), bly = blx, blz = blx, bhx = -blx, bhy = -blx, bhz = -blx;
+    float kx[2], ky[2], kz[2];
+    float blx = __builtin_huge_valf(), bly = blx, blz = blx, bhx = -blx, bhy = -blx, bhz = -blx;
 #pragma unroll
-        for (int u = 0; u < SU; u++) {
-            const int gi = min(g0 + grp * SU + u, r - 1);
-            const float3 k = pencil_sink(v, sc, w.first + gi, cx.invcpd);
-            kx[u] = k.x;
-            ky[u] = k.y;
-            kz[u] = k.z;
-            blx = fminf(blx, k.x);
-            bly = fminf(bly, k.y);
-            blz = fminf(blz, k.z);
-            bhx = fmaxf(bhx, k.x);
-            bhy = fmaxf(bhy, k.y);
-            bhz = fmaxf(bhz, k.z);
-        }
-        // The pass's box over all four groups: the tile mode is wave-uniform.
-        blx = wave_min(blx);
-        bly = wave_min(bly);
-        blz = wave_min(blz);
-        bhx = wave_max(bhx);
-        bhy = wave_max(bhy);
-        bhz = wave_max(bhz);
-        float hx[SU], hy[SU], hz[SU], lx[SU], ly[SU], lz[SU], hw[SU];
+    for (int u = 0; u < 2; u++) {  // (an odd r repeats its last sink in the free slot, not stored)
+        const float3 k = pencil_sink(v, sc, w.first + min(slot + u * L, r - 1), cx.invcpd);
+        kx[u] = k.x;
+        ky[u] = k.y;
+        kz[u] = k.z;
+        blx = fminf(blx, k.x);
+        bly = fminf(bly, k.y);
+        blz = fminf(blz, k.z);
+        bhx = fmaxf(bhx, k.x);
+        bhy = fmaxf(bhy, k.y);
+        bhz = fmaxf(bhz, k.z);
+    }
+    blz = wave_min(blz);
+    bhz = wave_max(bhz);
+    const SinkBox kbox = {wave_min(blx), wave_min(bly), wave_max(bhx), wave_max(bhy), blz, bhz, blz, bhz};
+    double h[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+    const int W = v.W, full64 = kWave / G;
+    int modes = 0, p = 0;
+    for (int y = 0; y < W; y++) {
+        const int st = rows.start_of(y), n = rows.count_of(y);
+        const double yo = (double)(y - v.R) * cx.invcpd;
+        float kyy[2];
 #pragma unroll
-        for (int u = 0; u < SU; u++) hx[u] = hy[u] = hz[u] = lx[u] = ly[u] = lz[u] = hw[u] = 0.f;
-        for (int y = 0; y < W; y++) {
-            const int si = ilist[s * W + y];
-            const int st = src_set_start[si];
-            const int n = src_set_count[si];
-            const double yo = (double)(y - v.R) * cx.invcpd;
-            float kyy[SU];
-#pragma unroll
-            for (int u = 0; u < SU; u++) kyy[u] = (float)((double)ky[u] - yo);
-            const float sly = (float)((double)bly - yo), shy = (float)((double)bhy - yo);
-            const int nblk = (n + kWave - 1) / kWave;
-            for (int b0 = 0; b0 < nblk; b0 += TC) {
-                const int b1 = min(nblk, b0 + TC);
-                float tx[SU], ty[SU], tz[SU], tw[SU];
-#pragma unroll
-                for (int u = 0; u < SU; u++) tx[u] = ty[u] = tz[u] = tw[u] = 0.f;
-                for (int b = b0; b < b1; b++) {
-                    const int64_t gb = (int64_t)st / kWave + b;
-                    const int mode =
-                        tile_mode<SOFT>(cx, box_gap2(blx, sly, blz, bhx, shy, bhz, box[2 * gb], box[2 * gb + 1]));
-                    if constexpr (CENSUS) {
-                        const uint64_t pairs =
-                            (uint64_t)min(kGroups * SU, r - g0) * (uint64_t)min(kWave, n - b * kWave);
-                        census_add(cen, mode, pairs);
-                        cen.tail += pairs;
-                    }
-                    // The block's 64 sources (padding included: exact zeros),
-                    // 16 at a time on the group's lanes.
-                    const float4 *bp = src + st + b * kWave + gl;
-#pragma unroll
-                    for (int c = 0; c < kGroups; c++) {
-                        const float4 sv = bp[c * kGroupLanes];
-                        if (mode == kNoDensity) {
-#pragma unroll
-                            for (int u = 0; u < SU; u++)
-                                pair_box<SOFT, kNoDensity>(sv.x, sv.y, sv.z, kx[u], kyy[u], kz[u], cx.pc, tx[u],
-                                                           ty[u], tz[u], tw[u]);
-                        } else if (mode == kDensity) {
-#pragma unroll
-                            for (int u = 0; u < SU; u++)
-                                pair_box<SOFT, kDensity>(sv.x, sv.y, sv.z, kx[u], kyy[u], kz[u], cx.pc, tx[u], ty[u],
-                                                         tz[u], tw[u]);
-                        } else {
-#pragma unroll
-                            for (int u = 0; u < SU; u++)
-                                pair_box<SOFT, kExact>(sv.x, sv.y, sv.z, kx[u], kyy[u], kz[u], cx.pc, tx[u], ty[u],
-                                                       tz[u], tw[u]);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < SU; u++) {
-                    merge(hx[u], lx[u], tx[u]);
-                    merge(hy[u], ly[u], ty[u]);
-                    merge(hz[u], lz[u], tz[u]);
-                    hw[u] += tw[u];
-                }
+        for (int u = 0; u < 2; u++) kyy[u] = (float)((double)ky[u] - yo);
+        const int nblk = (n + kWave - 1) / kWave;
+        for (int b = 0; b < nblk; b++, p++) {
+            if ((p & (kWave - 1)) == 0) modes = block_forms<SOFT, false>(cx, v, rows, kbox, p, lane);
+            const int mode = __builtin_amdgcn_readlane(modes, p & (kWave - 1)) & 3;
+            const int cnt = min(kWave, n - b * kWave);
+            if constexpr (CENSUS) {
+                census_add(cen, mode, (uint64_t)r * (uint64_t)cnt);
+                cen.tail += (uint64_t)r * (uint64_t)cnt;
             }
-        }
+            const float4 *bp = src + st + b * kWave;
+            const int full = cnt == kWave ? full64 : cnt / G;
+            float tx[2] = {0.f, 0.f}, ty[2] = {0.f, 0.f}, tz[2] = {0.f, 0.f}, tw[2] = {0.f, 0.f};
+            if (mode == kNoDensity)
+                tail_block<SOFT, kNoDensity>(bp, cnt, G, full, grp, kx, kyy, kz, cx.pc, tx, ty, tz, tw);
+            else if (mode == kDensity)
+                tail_block<SOFT, kDensity>(bp, cnt, G, full, grp, kx, kyy, kz, cx.pc, tx, ty, tz, tw);
+            else
+                tail_block<SOFT, kExact>(bp, cnt, G, full, grp, kx, kyy, kz, cx.pc, tx, ty, tz, tw);
 #pragma unroll
-        for (int u = 0; u < SU; u++) {
-            group_two_sum(hx[u], lx[u]);
-            group_two_sum(hy[u], ly[u]);
-            group_two_sum(hz[u], lz[u]);
-            const double ws = group_sum((double)hw[u]);  // (an FP64 lane sum spills at S = 2)
-            const int gi = g0 + grp * SU + u;
-            if (gl == 0 && gi < r) {
-                NF_GLOBAL double *o = out + 4 * (int64_t)(base + gi);
-                o[0] = (double)hx[u] + (double)lx[u];
-                o[1] = (double)hy[u] + (double)ly[u];
-                o[2] = (double)hz[u] + (double)lz[u];
-                o[3] = ws;
+            for (int u = 0; u < 2; u++) {
+                h[u][0] += (double)tx[u];
+                h[u][1] += (double)ty[u];
+                h[u][2] += (double)tz[u];
+                h[u][3] += (double)tw[u];
             }
         }
     }
+    for (int m = G; m > 1;) {  // groups [half, m) onto [0, m - half)
+        const int half = (m + 1) / 2;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const double o = __shfl(h[u][c], lane + half * L);
+                if (g + half < m) h[u][c] += o;
+            }
+        m = half;
+    }
+    if (g > 0) return;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        if (slot + u * L >= r) continue;
+        NF_GLOBAL double *o = out + 4 * (int64_t)(base + slot + u * L);
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = h[u][c];
+    }
 }
-
-constexpr int kRemSinks = 2;  // sinks per 16-lane group per pass of a short tail
 
 // Occupancy target WPE (waves per SIMD): more resident waves hide the v_rsq
 // and scalar-load latencies, as long as the tile loops' registers fit.  The
 // most waves at which each (pair form, sinks per lane) compiled with no VGPR
-// spills for gfx950 (6 waves: 80 VGPRs; 5: 96; 4: 128; 2: 256); the single
-// spline and Plummer forms keep 4 waves at S = 4, which measured faster than
-// 5.  With FP64 tile accumulation the S = 1 forms spill a few words in their
-// item set-up, outside the tile loops, at no measured cost.
-constexpr int batched_waves_per_eu(int soft, int s) {
-    switch (soft) {
-        case NF_SOFT_SINGLE_SPLINE: return s == 4 ? 4 : 6;
-        case NF_SOFT_PLUMMER: return s == 4 ? 4 : 5;
-        case NF_SOFT_CUBIC_SPLINE: return s == 1 ? 5 : s == 2 ? 4 : 2;
-        default: return s == 4 ? 5 : 6;  // cubic Plummer
-    }
-}
+// spills in its tile loops for gfx950 (6 waves: 80 VGPRs; 4: 128); S = 4 keeps
+// 4 waves, which measured faster than 5.
+constexpr int batched_waves_per_eu(int /*soft*/, int s) { return s == 4 ? 4 : 6; }
 
 }  // namespace
 
@@ -1261,13 +1262,22 @@ namespace {
 // Persistent kernel: every wave pops items (of any SIC of the group) until
 // the queue is empty.  CENSUS: count the pair interactions of each pair form
 // into census (the diagnostic instantiations; the results are the same).
-// counter[0] is the queue; nitems < 0 means a list of at most -nitems items
-// whose length the prologue wrote into counter[1]; a census build adds its
-// counts into the four uint64 at counter + kCensusOffset.  One queue for
-// the whole grid: dealing the list to one queue per XCD, in interleaved
-// chunks of 8 to 128 consecutive items (which share source pencils), was
-// measured 11% slower.
-constexpr int kCensusOffset = 16;  // int32 units: 64 bytes into the counter's slot
+// nitems < 0 means a list of at most -nitems items whose length the prologue
+// wrote into counter[1]; a census build adds its counts into the four uint64
+// at counter + kCensusOffset.
+//
+// Wave g takes item g first, without an atomic, then pops the rest of the list
+// from queue g mod kQueues, whose items are every kQueues-th one.  Atomics on
+// one address retire one per 11.7 ns (28 cycles) whatever the grid, so a
+// single queue held 6,144 waves for 72 us at their first pop and a list of
+// short items (133,000 in a launch group of sparse cells) for 1.6 ms; 16
+// queues on cache lines of their own pop 16 times as fast.  Waves do not look
+// into other queues when theirs is empty: the queues deal the cost-sorted list
+// out item by item, so they end within about an item of each other.  (Dealing
+// it to one queue per XCD in chunks of 8 to 128 consecutive items, which share
+// source pencils, measured 11% slower.)
+constexpr int kCensusOffset = kCensusBytes / 4;  // int32 units
+constexpr int kQueueOffset = kQueueBytes / 4, kQueueStride = kQueueLine / 4;
 template <int SOFT, int S, int WPE, bool CENSUS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_batched(
     BatchCtx cx, const SicView *__restrict__ views, const WorkItem *__restrict__ items, int32_t nitems,
@@ -1275,10 +1285,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
     const int lane = threadIdx.x & (kWave - 1);
     if (nitems < 0) nitems = min(-nitems, *cptr<int32_t>(counter + 1));
     Census cen = {{0, 0, 0}, 0};
+    const int wpw = blockDim.x / kWave, nwaves = gridDim.x * wpw;
+    const int g = __builtin_amdgcn_readfirstlane(blockIdx.x * wpw + (int)(threadIdx.x / kWave));
+    const int nq = min(kQueues, nwaves), q = g % nq;  // (a grid of fewer waves serves as many queues)
+    int it = g;
     for (;;) {
-        int it = 0;
-        if (lane == 0) it = atomicAdd(counter, 1);
-        it = __builtin_amdgcn_readfirstlane(it);
         if (it >= nitems) {
             if (CENSUS && lane == 0) {
                 unsigned long long *census = reinterpret_cast<unsigned long long *>(counter + kCensusOffset);
@@ -1293,16 +1304,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
         const SicView v = cptr<SicView>(views)[w.kind_sic >> 2];
         if (kind == 0) full_item<SOFT, S, CENSUS>(cx, v, w, lane, cen);
         else if (kind == 2) full_item<SOFT, 1, CENSUS>(cx, v, w, lane, cen);
-        else rem_item<SOFT, kRemSinks, CENSUS>(cx, v, w, lane, cen);
+        else tail_item<SOFT, CENSUS>(cx, v, w, lane, cen);
+        int j = 0;
+        if (lane == 0) j = atomicAdd(counter + kQueueOffset + q * kQueueStride, 1);
+        it = nwaves + __builtin_amdgcn_readfirstlane(j) * nq + q;
     }
 }
 
 // The batched launch's prologue (a fill kernel, so that it can sit in a
-// captured graph): clears the queue counter and, for a census build, the
-// census; for a device-planned list, copies its length into counter[1], or
+// captured graph): clears the queues and, for a census build, the census; for a device-planned list, copies its length into counter[1], or
 // 0 when the group holds a cell outside its slab.
 __global__ void k_zero_counter(int32_t *c, const int32_t *dnitems, const int32_t *dbad, int census) {
-    c[0] = 0;
+    const int t = threadIdx.x;
+    if (t < kQueues) c[kQueueOffset + t * kQueueStride] = 0;
+    if (t != 0) return;
     if (dnitems) c[1] = (dbad && *dbad != 0) ? 0 : *dnitems;
     if (census) {
         unsigned long long *cs = reinterpret_cast<unsigned long long *>(c + kCensusOffset);
@@ -1516,8 +1531,8 @@ static int launch_batched_k(const BatchCtx &cx, const TileShape &ts, const SicVi
     int grid = std::max(1, ncu) * blocks_per_cu;
     const int need = (nitems + wpw - 1) / wpw;
     if (grid > need) grid = std::max(1, need);
-    static_assert(kCensusOffset * 4 == kCensusBytes && kCensusBytes + 32 <= 256, "census inside the counter's slot");
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, st, counter, dnitems, dbad, CENSUS ? 1 : 0);
+    static_assert(kCensusBytes + 32 <= kQueueBytes && kQueues <= kWave, "census before the queues, one lane per queue");
+    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(kWave), 0, st, counter, dnitems, dbad, CENSUS ? 1 : 0);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, st, cx, views, items, dnitems ? -nitems : nitems, counter);
     return (int)hipGetLastError();
 }

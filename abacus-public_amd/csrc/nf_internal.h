@@ -28,10 +28,12 @@ void par_memcpy(void *dst, const void *src, size_t bytes);
 // `first` within sink pencil `sinkset`.  kind 0: register tile of 64*S sinks,
 // sinks on lanes; kind 2: one-wave tile of up to 64 sinks on the lanes (a
 // pencil's tail; lanes past nsink idle); kind 1: a short tail (fewer than
-// kTailLanes sinks), sources on the lanes.
-// Measured on uniform and clustered boxes (thresholds 1-60): 32 is fastest
-// on both, 3-4% ahead of 53 on a clustered box, 1.5% on a uniform one.
-constexpr int kTailLanes = 32;  // below this many sinks a tail is cheaper with sources on the lanes
+// kTailLanes sinks), two sinks to a lane and the sources dealt to groups of
+// lanes.  A one-wave tile takes one pair instruction per source; a short tail
+// of r sinks two per 64 / ceil(r / 2) sources, which is fewer up to 42 sinks
+// (three groups of lanes) and as many above.  Measured: 512^3 slabs, kernel
+// 14.04 ms with the line at 32 sinks, 13.86 ms at 43 and at 64.
+constexpr int kTailLanes = 43;
 
 struct WorkItem {
     int32_t sinkset;
@@ -159,12 +161,15 @@ int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, con
 // One persistent launch over the work items of a group of SICs.  With
 // dnitems (device memory) non-null the list holds *dnitems items and nitems
 // is only its bound; with dbad non-null and *dbad != 0 the kernel does
-// nothing.  counter names a 256-byte slot: the queue counter, the device
-// list's length and, with census, four uint64 at byte 64 (kCensusBytes)
-// receiving the pair interactions computed in each pair form (unsoftened,
-// with density, softened) and, in the fourth, those of short tails (also
-// counted by form), by a diagnostic build of the kernel.
+// nothing.  counter names a slot of kCounterBytes: the device list's length
+// (int32 1), with census four uint64 at kCensusBytes receiving the pair
+// interactions computed in each pair form (unsoftened, with density, softened)
+// and, in the fourth, those of short tails (also counted by form), by a
+// diagnostic build of the kernel; and kQueues queue counters from kQueueBytes,
+// kQueueLine bytes apart.
 constexpr int kCensusBytes = 64;
+constexpr int kQueues = 16, kQueueBytes = 256, kQueueLine = 256;
+constexpr int kCounterBytes = kQueueBytes + kQueues * kQueueLine;
 int launch_batched(const SicView *views, int cpd, int softening, const PairConst &pc, const TileShape &ts,
                    const WorkItem *items, int32_t nitems, int32_t *counter, void *stream,
                    const int32_t *dnitems = nullptr, const int32_t *dbad = nullptr, bool census = false);

@@ -484,7 +484,7 @@ void task_rows(const Task &t, uint64_t *r0, uint64_t *r1) {
 
 // Device bytes a SIC adds to a group (plan + work + host-mode slabs).
 size_t task_bytes(const nf_sic &s, int path, int32_t n_chunks) {
-    size_t b = plan_layout(s, 0, n_chunks).total + work_layout(s, path, 0).total + sizeof(SicView) + 256;
+    size_t b = plan_layout(s, 0, n_chunks).total + work_layout(s, path, 0).total + sizeof(SicView) + kCounterBytes;
     b += ((size_t)s.NSinkBlocks + 2 * (size_t)s.NSinkSets) * sizeof(WorkItem);  // at most one item per block + tails
     if (s.mem == NF_MEM_HOST) {
         for (int c = 0; c < s.nfwidth; c++) b += align_up(12 * (size_t)s.Nslab[c], 256);
@@ -1118,7 +1118,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         }
     }
     const size_t o_counter = align_up(o_items + std::max<size_t>(items_total, 256), 256);
-    size_t plan_total = align_up(o_counter + 256, 256);
+    size_t plan_total = align_up(o_counter + kCounterBytes, 256);
     std::vector<PlanLayout> PL(n);
     for (int i = 0; i < n; i++) {
         PL[i] = plan_layout(g[i]->sic, plan_total,
@@ -1383,7 +1383,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     unsigned long long *census = nullptr;  // batched path: interactions per pair form (device)
     if (path == NF_PATH_BATCHED) {
         int32_t *counter = reinterpret_cast<int32_t *>(pd + o_counter);
-        if (rt.params.census)  // in the counter's 256-byte slot
+        if (rt.params.census)  // in the counter's slot
             census = reinterpret_cast<unsigned long long *>(pd + o_counter + kCensusBytes);
         // A device-planned group's list lengths and bad cells are in its
         // shared planning area.
@@ -2231,7 +2231,7 @@ NoallocLayout noalloc_layout(const nf_sic &s) {
     L.items_max = (size_t)s.NSinkBlocks + (size_t)s.NSinkSets;
     L.o_items = align_up(sizeof(SicView), 256);
     L.o_counter = align_up(L.o_items + sizeof(WorkItem) * std::max<size_t>(L.items_max, 1), 256);
-    L.o_plan = L.o_counter + 256;
+    L.o_plan = align_up(L.o_counter + kCounterBytes, 256);
     L.plan = plan_layout(s, L.o_plan, count_coadd_chunks(s));
     L.image = L.o_plan + L.plan.total;
     L.o_work = align_up(L.image, 256);
