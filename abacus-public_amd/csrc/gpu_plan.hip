@@ -81,24 +81,28 @@ __device__ __forceinline__ uint64_t sink_pencil_sources(const GPlanIn &in, int j
 }
 
 // The work items of a pencil of n sinks (meeting nsrc sources) for register
-// tile S, as the runtime's host build_items makes them: `full` tiles of 64 S
+// tile S, as the runtime's host for_each_run makes them: `full` tiles of 64 S
 // sinks (kind 0), then one-wave tiles (kind 2) while at least kTailLanes
 // sinks remain -- q of 64 sinks and, if the rest s is at least kTailLanes,
 // one of s -- then one short tail of s sinks (kind 1) if 0 < s < kTailLanes.
 // A pencil whose register tile would cost more than split_cost takes no
-// register tiles: one-wave tiles from its first sink.
+// register tiles: one-wave tiles from its first sink.  If y_split, each of its
+// one-wave tiles is W items (kind 3), one per source pencil (ny = W, else 1).
 struct ItemSplit {
-    int full, tile, n2, q, s, tail;
-    __device__ ItemSplit(int n, int S, uint64_t nsrc, uint64_t split_cost) {
+    int full, tile, n2, q, s, tail, ny;
+    __device__ ItemSplit(int n, int S, uint64_t nsrc, const GPlanIn &in) {
+        const uint64_t split_cost = in.split_cost[S == 1 ? 0 : S == 2 ? 1 : 2];
+        ny = y_split(nsrc, in.y_cost) ? in.W : 1;
         tile = kB * S;
-        full = (S > 1 && (uint64_t)tile * nsrc > split_cost) ? 0 : n / tile;
+        full = ny > 1 || (S > 1 && (uint64_t)tile * nsrc > split_cost) ? 0 : n / tile;
         const int r = n - full * tile;
         q = r / kB;
         s = r - q * kB;
-        n2 = q + (s >= kTailLanes ? 1 : 0);
+        n2 = (q + (s >= kTailLanes ? 1 : 0)) * ny;
         tail = (s > 0 && s < kTailLanes) ? 1 : 0;
     }
     __device__ int count() const { return full + n2 + tail; }
+    __device__ uint64_t one_wave_cost(uint64_t nsrc) const { return kB * nsrc / (uint64_t)ny; }
 };
 
 // 1/8-octave cost buckets, longest first (cost 0 last).
@@ -172,7 +176,7 @@ __device__ void plan_a(const GPlanIn &in, GPlanTotals *tot, int32_t *group, int 
         sblk = (uint64_t)nblocks(n);
         ch = (uint64_t)nblocks(row[k].count);  // pencil k starts with cell z = k: its chunks are that cell's
         const uint64_t nsrc = sink_pencil_sources(in, j, k);
-        for (int ti = 0; ti < 3; ti++) it[ti] = (uint64_t)ItemSplit(n, 1 << ti, nsrc, in.split_cost[ti]).count();
+        for (int ti = 0; ti < 3; ti++) it[ti] = (uint64_t)ItemSplit(n, 1 << ti, nsrc, in).count();
         const int bin = n < 64 ? 0 : n < 256 ? 1 : n < 1024 ? 2 : 3;
         for (int i = 0; i < 4; i++) occ[i] = bin == i ? (uint64_t)n : 0;
         d = (uint64_t)n * nsrc;
@@ -252,10 +256,10 @@ __device__ void plan_b1(const GPlanIn &in, const GPlanOut &out, int bid) {
                 const uint64_t nsrc = sink_pencil_sources(in, j, k);
                 for (int ti = 0; ti < 3; ti++) {
                     if (!out.items[ti]) continue;
-                    const ItemSplit sp(n, 1 << ti, nsrc, in.split_cost[ti]);
+                    const ItemSplit sp(n, 1 << ti, nsrc, in);
                     int32_t *h = lh + ti * kPlanBuckets;
                     if (sp.full) atomicAdd(h + cost_bucket((uint64_t)sp.tile * nsrc), sp.full);
-                    if (sp.n2) atomicAdd(h + cost_bucket((uint64_t)kB * nsrc), sp.n2);
+                    if (sp.n2) atomicAdd(h + cost_bucket(sp.one_wave_cost(nsrc)), sp.n2);
                     if (sp.tail) atomicAdd(h + 3 * kPlanBuckets + cost_bucket((uint64_t)sp.s * nsrc), 1);
                 }
             }
@@ -320,10 +324,10 @@ __device__ void place_items(const GPlanIn &in, const GPlanOut &out, const int32_
     const uint64_t nsrc = n > 0 ? sink_pencil_sources(in, s / in.cpd, s % in.cpd) : 0;
     int bk[3][3], lo[3][3];  // per tile: bucket and local offset of the full, one-wave and tail runs
     for (int ti = 0; ti < 3; ti++) {
-        const ItemSplit sp(n, 1 << ti, nsrc, in.split_cost[ti]);
+        const ItemSplit sp(n, 1 << ti, nsrc, in);
         const bool on = out.items[ti] != nullptr && n > 0;
         bk[ti][0] = cost_bucket((uint64_t)sp.tile * nsrc);
-        bk[ti][1] = cost_bucket((uint64_t)kB * nsrc);
+        bk[ti][1] = cost_bucket(sp.one_wave_cost(nsrc));
         bk[ti][2] = cost_bucket((uint64_t)sp.s * nsrc);
         int32_t *h = lc + ti * kPlanBuckets;
         lo[ti][0] = on && sp.full ? atomicAdd(h + bk[ti][0], sp.full) : 0;
@@ -339,7 +343,7 @@ __device__ void place_items(const GPlanIn &in, const GPlanOut &out, const int32_
     for (int ti = 0; ti < 3; ti++) {
         WorkItem *items = out.items[ti];
         if (!items) continue;
-        const ItemSplit sp(n, 1 << ti, nsrc, in.split_cost[ti]);
+        const ItemSplit sp(n, 1 << ti, nsrc, in);
         const int32_t *base = lc + ti * kPlanBuckets, *tbase = lc + (3 + ti) * kPlanBuckets;
         const int64_t M = mt[ti], T = mt[3 + ti];
         if (sp.full) {
@@ -350,8 +354,11 @@ __device__ void place_items(const GPlanIn &in, const GPlanOut &out, const int32_
         const int f = sp.full * sp.tile;
         if (sp.n2) {
             const int p = boff[ti][bk[ti][1]] + base[bk[ti][1]] + lo[ti][1];
-            for (int i = 0; i < sp.n2; i++)
-                items[interleave_pos(false, p + i, M, T)] = WorkItem{s, f + i * kB, i < sp.q ? kB : sp.s, 2 + sic4};
+            for (int i = 0; i < sp.n2; i++) {
+                const int t = i / sp.ny, y = i % sp.ny;  // (a tile's source pencils next to each other)
+                items[interleave_pos(false, p + i, M, T)] =
+                    WorkItem{s, f + t * kB, (t < sp.q ? kB : sp.s) + 256 * y, (sp.ny > 1 ? 3 : 2) + sic4};
+            }
         }
         if (sp.tail) {
             const int p = boff[3 + ti][bk[ti][2]] + tbase[bk[ti][2]] + lo[ti][2];

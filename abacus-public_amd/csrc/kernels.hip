@@ -577,8 +577,10 @@ __global__ __launch_bounds__(64) void k_plain(DevPlan pl, PairConst pc, const fl
 // Addresses of the W partials of the sinks of cell (j_low + j, z): the cell is
 // at position c of pencil k = z - c (mod cpd).  Returns the cell's slab start
 // and count; base[c] is the padded slot of its first particle in pencil k.
+// and, if planes, split[c] the first of the cell's particles (its own numbering)
+// whose partial in pencil k is not spread over the source pencils' planes.
 __device__ __forceinline__ void partial_slots(const DevPlan &pl, int j, int z, int64_t *base, uint32_t *cstart,
-                                              int *cn) {
+                                              int *cn, bool planes = false, int *split = nullptr) {
     const int Nk = pl.Nk, W = pl.W, cpd = pl.cpd;
     const nf_sink_plan &own = pl.sink_plan[j * Nk + z];  // pencil k = z starts with cell z
     *cstart = own.cell[0].start;
@@ -591,6 +593,11 @@ __device__ __forceinline__ void partial_slots(const DevPlan &pl, int j, int z, i
         int off = 0;
         for (int c2 = 0; c2 < c; c2++) off += pk.cell[c2].N;
         base[c] = (int64_t)pl.sink_set_start[s] + off;
+        if (planes) {
+            uint64_t nsrc = 0;
+            for (int y = 0; y < W; y++) nsrc += (uint64_t)pl.src_set_count[pl.ilist[s * W + y]];
+            split[c] = y_split(nsrc, pl.y_cost) ? tile_sinks(pl.sink_set_count[s]) - off : 0;
+        }
     }
 }
 
@@ -651,19 +658,30 @@ __device__ __forceinline__ void coadd_chunk_f64(const DevPlan &pl, const double 
     const int cell = pl.coadd_chunk[2 * q], first = pl.coadd_chunk[2 * q + 1];
     const int j = cell / pl.Nk, z = cell % pl.Nk;
     int64_t base[NF_MAX_WIDTH];
+    int split[NF_MAX_WIDTH];
     uint32_t cstart;
     int cn;
-    partial_slots(pl, j, z, base, &cstart, &cn);
+    const int64_t plane = pl.y_plane;
+    partial_slots(pl, j, z, base, &cstart, &cn, plane != 0, split);
     const int W = pl.W;
     const int i = first + lane;
     if (i >= cn) return;
     double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
     for (int c = 0; c < W; c++) {
         const double *p = part + 4 * (base[c] + i);
-        a0 += p[0];
-        a1 += p[1];
-        a2 += p[2];
-        a3 += p[3];
+        double h0 = p[0], h1 = p[1], h2 = p[2], h3 = p[3];
+        if (plane != 0 && i < split[c])
+            for (int y = 1; y < W; y++) {
+                const double *q = p + y * plane;
+                h0 += q[0];
+                h1 += q[1];
+                h2 += q[2];
+                h3 += q[3];
+            }
+        a0 += h0;
+        a1 += h1;
+        a2 += h2;
+        a3 += h3;
     }
     const float4 a = make_float4((float)(a0 * out_scale), (float)(a1 * out_scale), (float)(a2 * out_scale), (float)a3);
     acc[cstart + i] = apply_kick(a, kick, (int64_t)cstart + i);
@@ -744,11 +762,14 @@ __device__ __forceinline__ float pair_g(float r2, float f, const PairConst &pc) 
         return fminf(f3, fmaf(fmaf(pc.c1, f, pc.c2), r2, pc.c3));
     } else {
         // Cubic spline, u = r/e: f^3 beyond 2, below it e^-3 times a cubic in u
-        // (from 1 on, with the -1/(15 u^3) of the middle piece as -f^3/15).
+        // (from 1 on, with the -1/(15 u^3) of the middle piece as -f^3/15, and
+        // 8/3 - 3 u + 6/5 u^2 - u^3/6 about u = 3/2, where its terms are no
+        // larger than its values: about 0 they cancel to a 50th).
         // Selects, not branches: nearly every wave has lanes in each piece.  A
         // padding source (r2 = inf, f = 0) has u = NaN and takes f^3 = 0.
         const float u = r2 * f * pc.eps;
-        const float mid = fmaf(fmaf(fmaf((float)(-1.0 / 6.0), u, (float)(6.0 / 5.0)), u, -3.0f), u, (float)(8.0 / 3.0));
+        const float t = u - 1.5f;
+        const float mid = fmaf(fmaf(fmaf((float)(-1.0 / 6.0), t, 0.45f), t, -0.525f), t, (float)(73.0 / 240.0));
         const float in = fmaf(fmaf(0.5f, u, (float)(-6.0 / 5.0)), u * u, (float)(4.0 / 3.0));
         const bool outer = u >= 1.0f;
         const float soft = fmaf(outer ? mid : in, pc.c3, outer ? f3 * (float)(-1.0 / 15.0) : 0.0f);
@@ -998,15 +1019,17 @@ __device__ __forceinline__ void mixed_tile(int mlo, int mhi, const NF_CONST floa
 
 // Register tile: 64*S sinks of one pencil on the lanes; sources are wave
 // uniform and come through the scalar cache.
+// It meets source pencils [y0, y1); hsum: the lane's place in the wave's LDS
+// accumulators, 4 S of them 64 apart.
 template <int SOFT, int S, bool CENSUS>
-__device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int lane,
-                                          Census &cen) {
+__device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int nsink, int y0,
+                                          int y1, double *hsum, int lane, Census &cen) {
     const NF_CONST float4 *src = cptr<float4>(v.sources4);
     NF_GLOBAL double *out = (NF_GLOBAL double *)v.partial;
     const int s = w.sinkset;
     const int base = cptr<int32_t>(v.sink_set_start)[s] + w.first;
     const SourceRows rows = source_rows(v, s, lane);
-    const int nsink = w.nsink;  // 64*S, or fewer for a masked tail tile
+    // nsink: 64*S, or fewer for a masked tail tile
     const uint64_t n_lo = (uint64_t)min(nsink, kWave * (S / 2)), n_hi = (uint64_t)nsink - n_lo;  // sinks per half
     const SinkCells sc = sink_cells(v, s);
     float kx[S], ky[S], kz[S];
@@ -1046,20 +1069,23 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
         bhz0 = wave_max(bhz0);
     }
 
-    // Each block's FP32 tile sum joins an FP64 partial: a convert and an add
-    // per component, which gfx950 issues at the FP32 rate (a TwoSum merge
+    // Each block's FP32 tile sum joins an FP64 sum: a convert and an add per
+    // component, which gfx950 issues at nearly the FP32 rate (a TwoSum merge
     // into an FP32 (hi, lo) pair is 7 instructions and carries fewer bits).
     // The FOF density w too: in a dense halo a sink meets thousands of pairs
-    // within b, and one FP32 running sum of them drifts by ~1e-5.
-    double hx[S], hy[S], hz[S], hw[S];
-#pragma unroll
-    for (int u = 0; u < S; u++) hx[u] = hy[u] = hz[u] = hw[u] = 0.0;
-
+    // within b, and one FP32 running sum of them drifts by ~1e-5.  The FP64
+    // sums are one source pencil's; the pencils' are added up in LDS, whose
+    // registers the tile loop has no room for.
     const SinkBox kbox = {blx, bly, bhx, bhy, blz0, bhz0, blz1, bhz1};
-    const int W = v.W;
-    int modes = 0, p = 0;  // p: blocks done; lane i: forms of block (p & ~63) + i
-    for (int y = 0; y < W; y++) {
+    int p = 0;  // the item's blocks: p next, counted from source pencil 0
+#pragma unroll
+    for (int y = 0; y < NF_MAX_WIDTH; y++) p = y < y0 ? rows.pre[y + 1] : p;
+    int modes = 0, pm0 = p;  // lane i: forms of block pm0 - 64 + i
+    for (int y = y0; y < y1; y++) {
         const int st = rows.start_of(y), n = rows.count_of(y);
+        double hx[S], hy[S], hz[S], hw[S];
+#pragma unroll
+        for (int u = 0; u < S; u++) hx[u] = hy[u] = hz[u] = hw[u] = 0.0;
         // Source y + (y-R)/cpd == sink y - (y-R)/cpd on the other side; the
         // cell-centre offset is formed in FP64.
         const double yo = (double)(y - v.R) * cx.invcpd;
@@ -1071,8 +1097,11 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
             // Lane i decides the pair forms of block i of the item's source
             // blocks (64 per pass): one vector pass instead of a wave-uniform
             // box test and a dependent box load per block.
-            if ((p & (kWave - 1)) == 0) modes = block_forms<SOFT, (S > 1)>(cx, v, rows, kbox, p, lane);
-            const int pm = __builtin_amdgcn_readlane(modes, p & (kWave - 1));
+            if (p == pm0) {
+                modes = block_forms<SOFT, (S > 1)>(cx, v, rows, kbox, p, lane);
+                pm0 += kWave;
+            }
+            const int pm = __builtin_amdgcn_readlane(modes, (p - pm0) & (kWave - 1));
             const int mlo = pm & 3, mhi = pm >> 2;
             const NF_CONST float4 *sp = src + st + b * kWave;
             const int cnt = min(kWave, n - b * kWave);
@@ -1092,15 +1121,23 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
                 hw[u] += (double)tw[u];
             }
         }
+#pragma unroll
+        for (int u = 0; u < S; u++) {
+            const double h[4] = {hx[u], hy[u], hz[u], hw[u]};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                double *const a = hsum + kWave * (4 * u + c);
+                *a = y == y0 ? h[c] : *a + h[c];
+            }
+        }
     }
+    if (y1 - y0 < v.W) out += y0 * v.y_plane;
 #pragma unroll
     for (int u = 0; u < S; u++) {
         if (lane + kWave * u >= nsink) continue;
         NF_GLOBAL double *o = out + 4 * (int64_t)(base + lane + kWave * u);
-        o[0] = hx[u];
-        o[1] = hy[u];
-        o[2] = hz[u];
-        o[3] = hw[u];
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = hsum[kWave * (4 * u + c)];
     }
 }
 
@@ -1283,6 +1320,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
     BatchCtx cx, const SicView *__restrict__ views, const WorkItem *__restrict__ items, int32_t nitems,
     int32_t *__restrict__ counter) {
     const int lane = threadIdx.x & (kWave - 1);
+    extern __shared__ double hsums[];  // per wave 4 S x 64: full_item's sums over the source pencils
+    double *const hsum = hsums + (threadIdx.x / kWave) * (4 * S * kWave) + lane;
     if (nitems < 0) nitems = min(-nitems, *cptr<int32_t>(counter + 1));
     Census cen = {{0, 0, 0}, 0};
     const int wpw = blockDim.x / kWave, nwaves = gridDim.x * wpw;
@@ -1302,9 +1341,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
         const WorkItem w = cptr<WorkItem>(items)[it];
         const int kind = w.kind_sic & 3;
         const SicView v = cptr<SicView>(views)[w.kind_sic >> 2];
-        if (kind == 0) full_item<SOFT, S, CENSUS>(cx, v, w, lane, cen);
-        else if (kind == 2) full_item<SOFT, 1, CENSUS>(cx, v, w, lane, cen);
-        else tail_item<SOFT, CENSUS>(cx, v, w, lane, cen);
+        if (kind == 0) {
+            full_item<SOFT, S, CENSUS>(cx, v, w, w.nsink, 0, v.W, hsum, lane, cen);
+        } else if (kind >= 2) {  // one-wave tiles, whole or against one source pencil
+            const int y = w.nsink >> 8;
+            full_item<SOFT, 1, CENSUS>(cx, v, w, w.nsink & 255, y, kind == 2 ? v.W : y + 1, hsum, lane, cen);
+        } else tail_item<SOFT, CENSUS>(cx, v, w, lane, cen);
         int j = 0;
         if (lane == 0) j = atomicAdd(counter + kQueueOffset + q * kQueueStride, 1);
         it = nwaves + __builtin_amdgcn_readfirstlane(j) * nq + q;
@@ -1522,8 +1564,9 @@ static int launch_batched_k(const BatchCtx &cx, const TileShape &ts, const SicVi
     // size only changes how the dispatcher places the persistent grid.
     const int wpw = ts.waves_per_wg == 1 || ts.waves_per_wg == 2 ? ts.waves_per_wg : 4;
     const int threads = kWave * wpw;
+    const size_t lds = sizeof(double) * 4 * S * threads;
     int blocks_per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, kern, threads, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, kern, threads, lds) != hipSuccess ||
         blocks_per_cu <= 0)
         blocks_per_cu = 1;
     if (ts.waves_per_cu > 0) blocks_per_cu = std::max(1, std::min(blocks_per_cu, ts.waves_per_cu / wpw));
@@ -1533,7 +1576,7 @@ static int launch_batched_k(const BatchCtx &cx, const TileShape &ts, const SicVi
     if (grid > need) grid = std::max(1, need);
     static_assert(kCensusBytes + 32 <= kQueueBytes && kQueues <= kWave, "census before the queues, one lane per queue");
     hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(kWave), 0, st, counter, dnitems, dbad, CENSUS ? 1 : 0);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, st, cx, views, items, dnitems ? -nitems : nitems, counter);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, st, cx, views, items, dnitems ? -nitems : nitems, counter);
     return (int)hipGetLastError();
 }
 

@@ -35,12 +35,28 @@ void par_memcpy(void *dst, const void *src, size_t bytes);
 // 14.04 ms with the line at 32 sinks, 13.86 ms at 43 and at 64.
 constexpr int kTailLanes = 43;
 
+// Kind 3: a one-wave tile against one of the W source pencils only, whose sums
+// go to that pencil's plane of the partials (see y_planes).
 struct WorkItem {
     int32_t sinkset;
     int32_t first;
-    int32_t nsink;
+    int32_t nsink;     // kind 3: nsink + 256 * source pencil
     int32_t kind_sic;  // kind + 4 * (index of the SIC in its launch group)
 };
+
+// Splitting over the source pencils.  A launch with little work per wave has
+// too few tiles to fill the GPU (a 64^3 box's SIC: 1,400 tiles for 6,144
+// waves), and its time is that of its longest tile.  There a pencil whose
+// one-wave tiles cost more than y_cost (sinks x sources) has each of them done
+// as W items, one per source pencil, and the partials get W planes of
+// `y_plane` doubles: the co-add adds the planes in source-pencil order.  A
+// whole tile sums each source pencil's FP64 sums apart and adds them in the
+// same order, so every sink's result is bitwise the same either way.  Sinks of
+// a pencil in its tiles (all but a short tail's):
+constexpr int32_t tile_sinks(int32_t n) {
+    return n % NF_BLOCK_SIZE < kTailLanes ? n - n % NF_BLOCK_SIZE : n;
+}
+constexpr bool y_split(uint64_t nsrc, uint64_t y_cost) { return NF_BLOCK_SIZE * nsrc > y_cost; }
 
 // A work list is two cost-sorted runs merged: the M register and one-wave
 // tiles, and the T short tails (kind 1) spread evenly through them, tail t
@@ -66,6 +82,7 @@ struct SicView {
     const void *sources4;           // padded source stream, float4, followed by 2 float4 boxes per block
     const void *box4;
     double *partial;                // 4 doubles per padded sink slot
+    int64_t y_plane;                // doubles between the source pencils' planes of it (0: one plane)
     int32_t W, R;
     int32_t aos;                    // 1: posstruct (x,y,z) per particle; 0: PosXYZ X|Y|Z
     int32_t pad;
@@ -98,6 +115,8 @@ struct DevPlan {
     int32_t W, R, cpd, Nk, j_width, j_low;
     int32_t n_coadd_chunks;
     int32_t max_src_blocks;  // padded blocks of the largest source pencil (INT32_MAX: not known)
+    int64_t y_plane;         // as SicView's
+    uint64_t y_cost;
     const GPlanTotals *dtot;
     const int32_t *dbad;
 };
@@ -228,6 +247,7 @@ struct GPlanIn {
     const nf_cellinfo *ci[NF_MAX_WIDTH];
     uint64_t nslab[NF_MAX_WIDTH];  // particles per slab: every planned cell must lie inside its slab
     uint64_t split_cost[3];        // per S = 1, 2, 4: register tiles above this cost become one-wave tiles
+    uint64_t y_cost;               // one-wave tiles above this cost are split over the source pencils
 };
 // Totals of phase A (device; atomically accumulated, so zeroed first).
 struct GPlanTotals {

@@ -157,6 +157,19 @@ struct PinBuf {
     }
 };
 
+// A run of like work items of a pencil: tiles of up to `step` sinks from
+// `first` to `end`.  Item i is tile i / ny against source pencil i % ny (ny > 1:
+// kind 3).
+struct ItemRun {
+    int32_t sinkset, first, step, end, kind_sic, ny;
+    int32_t key;  // counting-sort key: the cost's bucket, plus kItemBuckets for a tail
+    int count() const { return (end - first + step - 1) / step * ny; }
+    WorkItem item(int i) const {
+        const int f = first + i / ny * step;
+        return WorkItem{sinkset, f, std::min(step, end - f) + (ny > 1 ? 256 * (i % ny) : 0), kind_sic};
+    }
+};
+
 struct Worker {
     int id = 0;
     int device = 0;
@@ -174,6 +187,12 @@ struct Worker {
     uint64_t graphs_instantiated = 0, graphs_updated = 0;
     DevBuf plan, work, slabs;
     PinBuf pin_plan, pin_acc, pin_far;
+    // Work lists in the making (host-planned groups), kept so that a group does
+    // not fault their pages in again.
+    std::vector<uint32_t> sort_start;
+    std::vector<ItemRun> runs;
+    std::vector<uint64_t> nsrc;
+    std::vector<WorkItem> items[3];  // per sinks per lane: 1, 2, 4
     std::thread th;
     bool ready = false;
 };
@@ -450,14 +469,16 @@ struct WorkLayout {
     size_t o_sinks, o_src, o_part, o_far, total;
 };
 
-WorkLayout work_layout(const nf_sic &s, int path, size_t base) {
+// planes: of the batched path's partials (W where its tiles may be split over
+// the source pencils).
+WorkLayout work_layout(const nf_sic &s, int path, size_t base, int planes = 1) {
     WorkLayout L{};
     const size_t psink = (size_t)s.NSinkBlocks * NF_BLOCK_SIZE;
     const size_t psrc = (size_t)s.NSourceBlocks * NF_BLOCK_SIZE;
     L.o_sinks = base;  // the plain path's sink stream (the batched kernel reads the slab)
     L.o_src = align_up(L.o_sinks + (path == NF_PATH_BATCHED ? 0 : 16 * psink), 256);
     L.o_part = align_up(L.o_src + 16 * psrc + 32 * (size_t)s.NSourceBlocks, 256);
-    size_t end = align_up(L.o_part + psink * (path == NF_PATH_BATCHED ? 32 : 16), 256);
+    size_t end = align_up(L.o_part + psink * (path == NF_PATH_BATCHED ? 32 * (size_t)planes : 16), 256);
     L.o_far = end;  // host mode with a fused kick: the sink rows' far-field accelerations
     if (s.kick && s.mem == NF_MEM_HOST) end = align_up(end + 12 * (size_t)s.Nslab[s.nfradius], 256);
     L.total = end - base;
@@ -543,13 +564,22 @@ uint64_t queued_interactions(const Task &t) { return t.dp.on ? t.dp.interactions
 // The 1/8-octave bucket of an item's cost (sinks x sources), longest first:
 // bucket 0 holds the most expensive items, kItemBuckets - 1 the cheapest.
 constexpr int kItemBuckets = 1024;
-uint16_t cost_bucket(uint64_t cost) {
-    const uint64_t b = cost ? (uint64_t)std::floor(8.0 * std::log2((double)cost)) : 0;
-    return (uint16_t)(kItemBuckets - 1 - std::min<uint64_t>(b, kItemBuckets - 1));
+int cost_bucket(uint64_t cost) {
+    if (cost == 0) return kItemBuckets - 1;
+    // 8 log2 cost, rounded down: the exponent, and the eighth that the first 8
+    // mantissa bits lie in.
+    struct Eighths {
+        uint8_t of[256];
+        Eighths() {
+            for (int i = 0; i < 256; i++) of[i] = (uint8_t)std::floor(8.0 * std::log2(1.0 + i / 256.0));
+        }
+    };
+    static const Eighths eighths;
+    const double x = (double)cost;  // at least 1
+    uint64_t bits;
+    std::memcpy(&bits, &x, 8);
+    return kItemBuckets - 1 - std::min(8 * ((int)(bits >> 52) - 1023) + eighths.of[(bits >> 44) & 255], kItemBuckets - 1);
 }
-// Counting-sort key of an item: its bucket among the tiles, or kItemBuckets
-// plus its bucket among the short tails.
-int item_key(const WorkItem &w, uint16_t bucket) { return (int)bucket + ((w.kind_sic & 3) == 1 ? kItemBuckets : 0); }
 
 // The batched work list of one SIC, appended in sink-pencil order z then y
 // (pencils adjacent in y share 2R of their 2R+1 source pencils), with each
@@ -571,9 +601,42 @@ uint64_t tile_split_cost(int softening, int S, uint64_t interactions) {
                            (uint64_t)std::max(1, batched_kernel_waves(softening, S));
     return std::max<uint64_t>(kSplitMinCost, interactions / waves / 4);
 }
-// Calls emit(item, bucket) for each work item of the SIC, in list order.
+// The y_cost of a launch: in a launch below kYSplitWork a one-wave tile is
+// split over the source pencils if it costs more than an eighth of the work
+// per wave of the grid (6 waves per SIMD).  Measured, direct kernel: a SIC of a
+// 64^3 box 0.174 -> 0.084 ms, of a clustered 256^3 box (1.7e9 pairs) 0.78-0.91
+// -> 0.57-0.62 ms (a quarter of the work per wave 0.69-0.73, half 0.64-0.72,
+// the whole 0.74-0.81), two SICs of dense cells (4.4e9) 1.38 -> 1.21 ms.  At
+// the bound an ordinary tile (64 sinks x 1,350 sources) is half the line, and
+// launches above it have tiles enough.  A list built on the host takes longer
+// the more items it has, up to W times (10,000 pencils: 0.5 -> 1.1 ms), so
+// there only tiles above half the work per wave are split.  The planes take at
+// most kYSplitBytes.
+constexpr uint64_t kYSplitWork = 8000000000ull, kYSplitBytes = 512ull << 20;
+uint64_t y_split_cost(uint64_t interactions, bool host_list) {
+    if (interactions >= kYSplitWork) return UINT64_MAX;
+    return interactions / ((uint64_t)std::max(1, device_cu_count()) * 24) / (host_list ? 2 : 8);
+}
+// Work items of a SIC at most, where tiles may be split over the source pencils.
+uint64_t y_items_bound(const nf_sic &s) {
+    return (uint64_t)s.nfwidth * (uint64_t)s.NSinkBlocks + (uint64_t)s.NSinkSets;
+}
+// The partials' planes beyond the first, of SICs of nblocks padded sink blocks in all.
+uint64_t y_plane_bytes(uint64_t nblocks, int W) { return nblocks * NF_BLOCK_SIZE * 32 * (uint64_t)(W - 1); }
+
+// The sources that sink pencil k meets.
+uint64_t pencil_sources(const nf_sic &s, int k) {
+    const int W = s.nfwidth;
+    uint64_t n = 0;
+    for (int y = 0; y < W; y++) n += (uint64_t)s.SourceSetCount[s.SinkSourceInteractionList[W * k + y]];
+    return n;
+}
+// Calls emit(run) for each run of like work items of the SIC, in list order: a
+// pencil's tiles (kind 0, 2 or 3) and its short tail.  nsrcs (or null):
+// pencil_sources of every sink pencil, looked up in their own order.
 template <typename Emit>
-void for_each_item(const nf_sic &s, int S, int sic, uint64_t max_tile_cost, Emit &&emit) {
+void for_each_run(const nf_sic &s, int S, int sic, uint64_t max_tile_cost, uint64_t y_cost, const uint64_t *nsrcs,
+                  Emit &&emit) {
     const int tile = NF_BLOCK_SIZE * S;
     const int W = s.nfwidth;
     for (int z = 0; z < s.Nk; z++)
@@ -581,37 +644,56 @@ void for_each_item(const nf_sic &s, int S, int sic, uint64_t max_tile_cost, Emit
             const int k = j * s.Nk + z;
             const int n = s.SinkSetCount[k];
             if (n == 0) continue;
-            uint64_t nsrc = 0;
-            for (int y = 0; y < W; y++) nsrc += (uint64_t)s.SourceSetCount[s.SinkSourceInteractionList[W * k + y]];
+            const uint64_t nsrc = nsrcs ? nsrcs[k] : pencil_sources(s, k);
+            const int tiles = tile_sinks(n), ny = y_split(nsrc, y_cost) ? W : 1;
             int f = 0;
-            if (S > 1 && (uint64_t)tile * nsrc > max_tile_cost) {
-                const uint16_t b = cost_bucket((uint64_t)NF_BLOCK_SIZE * nsrc);
-                for (; f + NF_BLOCK_SIZE <= n; f += NF_BLOCK_SIZE) emit(WorkItem{k, f, NF_BLOCK_SIZE, 2 + 4 * sic}, b);
-            } else if (n >= tile) {
-                const uint16_t b = cost_bucket((uint64_t)tile * nsrc);
-                for (; f + tile <= n; f += tile) emit(WorkItem{k, f, tile, 0 + 4 * sic}, b);
+            if (ny == 1 && !(S > 1 && (uint64_t)tile * nsrc > max_tile_cost) && n >= tile) {
+                f = n / tile * tile;
+                emit(ItemRun{k, 0, tile, f, 0 + 4 * sic, 1, cost_bucket((uint64_t)tile * nsrc)});
             }
-            // The tail: one-wave tiles while they keep at least kTailLanes
-            // lanes busy, then the rest with sources on the lanes.
-            if (n - f >= kTailLanes) {
-                const uint16_t b = cost_bucket((uint64_t)NF_BLOCK_SIZE * nsrc);
-                while (n - f >= kTailLanes) {
-                    const int m = std::min(NF_BLOCK_SIZE, n - f);
-                    emit(WorkItem{k, f, m, 2 + 4 * sic}, b);
-                    f += m;
-                }
-            }
-            if (f < n) emit(WorkItem{k, f, n - f, 1 + 4 * sic}, cost_bucket((uint64_t)(n - f) * nsrc));
+            // One-wave tiles, the last of at least kTailLanes sinks, then the
+            // rest as a short tail.
+            if (f < tiles)
+                emit(ItemRun{k, f, NF_BLOCK_SIZE, tiles, (ny > 1 ? 3 : 2) + 4 * sic, ny,
+                             cost_bucket(NF_BLOCK_SIZE * nsrc / (uint64_t)ny)});
+            if (tiles < n)
+                emit(ItemRun{k, tiles, NF_BLOCK_SIZE, n, 1 + 4 * sic, 1,
+                             kItemBuckets + cost_bucket((uint64_t)(n - tiles) * nsrc)});
         }
 }
 
-void build_items(const nf_sic &s, int S, int sic, uint64_t max_tile_cost, std::vector<WorkItem> &items,
-                 std::vector<uint16_t> &bucket) {
-    for_each_item(s, S, sic, max_tile_cost, [&](const WorkItem &w, uint16_t b) {
-        items.push_back(w);
-        bucket.push_back(b);
-    });
-}
+// The counting sort of a work list, by cost bucket, of the tiles and of the
+// short tails apart: add() every run, begin(), then place() the same runs in
+// the same order.  A run's items are placed one after the other in its bucket's
+// stretch of its merged run (interleave_pos, stepped without divisions).
+struct ItemSort {
+    uint32_t *start;  // 2 kItemBuckets + 1, zeroed
+    int64_t M = 0, T = 0;
+    void add(const ItemRun &r) { start[r.key + 1] += (uint32_t)r.count(); }
+    size_t begin() {
+        for (int b = 0; b < 2 * kItemBuckets; b++) start[b + 1] += start[b];
+        M = start[kItemBuckets];
+        T = (int64_t)start[2 * kItemBuckets] - M;
+        return (size_t)(M + T);
+    }
+    void place(const ItemRun &r, WorkItem *out) {
+        const int cnt = r.count();
+        const int64_t at = start[r.key];
+        start[r.key] += (uint32_t)cnt;
+        if (r.key >= kItemBuckets) {  // a tail (cnt 1)
+            out[interleave_pos(true, at - M, M, T)] = r.item(0);
+            return;
+        }
+        // tails before tile `at`: at T / M (by a floating division, set right)
+        int64_t before = (int64_t)((double)(at * T) / (double)M), rem = at * T - before * M;
+        if (rem < 0) before--, rem += M;
+        if (rem >= M) before++, rem -= M;
+        for (int i = 0; i < cnt; i++) {
+            out[at + i + before] = r.item(i);
+            for (rem += T; rem >= M; rem -= M) before++;
+        }
+    }
+};
 
 int validate(const nf_sic &s) {
     if (s.nfradius < 0 || s.nfradius > NF_MAX_RADIUS || s.nfwidth != 2 * s.nfradius + 1)
@@ -638,14 +720,19 @@ int validate(const nf_sic &s) {
     if (s.mem != NF_MEM_HOST && s.mem != NF_MEM_DEVICE) return fail(NF_ERR_INVALID, "bad mem kind");
     // Every cell a plan names must lie inside its slab; the device gathers
     // index the slabs with these starts and counts.
+    const int W = s.nfwidth;
+    auto outside = [](const nf_cell_plan &cp, uint64_t nslab) {
+        return cp.N < 0 || (uint64_t)cp.start + (uint64_t)cp.N > nslab;
+    };
     for (int k = 0; k < s.NSinkSets; k++) {
         int64_t tot = 0;
-        for (int c = 0; c < s.nfwidth; c++) {
+        bool bad = false;
+        for (int c = 0; c < W; c++) {
             const nf_cell_plan &cp = s.SinkPlan[k].cell[c];
-            if (cp.N < 0 || (uint64_t)cp.start + (uint64_t)cp.N > s.Nslab[s.nfradius])
-                return fail(NF_ERR_INVALID, "sink plan cell outside its slab");
+            bad |= outside(cp, s.Nslab[s.nfradius]);
             tot += cp.N;
         }
+        if (bad) return fail(NF_ERR_INVALID, "sink plan cell outside its slab");
         if (tot != s.SinkSetCount[k]) return fail(NF_ERR_INVALID, "SinkSetCount disagrees with SinkPlan");
         if (s.SinkSetStart[k] % NF_BLOCK_SIZE != 0 || s.SinkSetStart[k] < 0 ||
             (int64_t)s.SinkSetStart[k] + (tot + NF_BLOCK_SIZE - 1) / NF_BLOCK_SIZE * NF_BLOCK_SIZE >
@@ -655,21 +742,22 @@ int validate(const nf_sic &s) {
     }
     for (int k = 0; k < s.NSourceSets; k++) {
         int64_t tot = 0;
-        for (int c = 0; c < s.nfwidth; c++) {
+        bool bad = false;
+        for (int c = 0; c < W; c++) {
             const nf_cell_plan &cp = s.SourcePlan[k].cell[c];
-            if (cp.N < 0 || (uint64_t)cp.start + (uint64_t)cp.N > s.Nslab[c])
-                return fail(NF_ERR_INVALID, "source plan cell outside its slab");
+            bad |= outside(cp, s.Nslab[c]);
             tot += cp.N;
         }
+        if (bad) return fail(NF_ERR_INVALID, "source plan cell outside its slab");
         if (tot != s.SourceSetCount[k]) return fail(NF_ERR_INVALID, "SourceSetCount disagrees with SourcePlan");
         if (s.SourceSetStart[k] % NF_BLOCK_SIZE != 0 || s.SourceSetStart[k] < 0 ||
             (int64_t)s.SourceSetStart[k] + (tot + NF_BLOCK_SIZE - 1) / NF_BLOCK_SIZE * NF_BLOCK_SIZE >
                 (int64_t)s.NSourceBlocks * NF_BLOCK_SIZE)
             return fail(NF_ERR_INVALID, "bad SourceSetStart");
     }
-    for (int i = 0; i < s.InteractionCount; i++)
-        if (s.SinkSourceInteractionList[i] < 0 || s.SinkSourceInteractionList[i] >= s.NSourceSets)
-            return fail(NF_ERR_INVALID, "interaction list entry out of range");
+    uint32_t largest = 0;  // (a negative entry is a large one)
+    for (int i = 0; i < s.InteractionCount; i++) largest = std::max(largest, (uint32_t)s.SinkSourceInteractionList[i]);
+    if (largest >= (uint32_t)s.NSourceSets) return fail(NF_ERR_INVALID, "interaction list entry out of range");
     // Each padded block must lie inside the padded range of the pencil it
     // names: the sink gather indexes the pencil by the block's offset.
     for (int b = 0; b < s.NSinkBlocks; b++) {
@@ -682,17 +770,16 @@ int validate(const nf_sic &s) {
     }
     // The co-add reads pencil k = z's first cell as cell z of the skewer:
     // the plans must follow the reference's pencil geometry.
-    for (int j = 0; j < s.j_width; j++)
-        for (int k = 0; k < s.Nk; k++) {
-            const nf_sink_plan &p = s.SinkPlan[j * s.Nk + k];
-            for (int c = 0; c + 1 < s.nfwidth; c++) {
-                const int z = (k + c) % s.cpd, z1 = (k + c + 1) % s.cpd;
-                const nf_sink_plan &a = s.SinkPlan[j * s.Nk + z], &b = s.SinkPlan[j * s.Nk + z1];
-                if (p.cell[c].start != a.cell[0].start || p.cell[c].N != a.cell[0].N ||
-                    p.cell[c + 1].start != b.cell[0].start || p.cell[c + 1].N != b.cell[0].N)
-                    return fail(NF_ERR_INVALID, "sink plans do not follow the pencil geometry");
+    for (int j = 0; j < s.j_width; j++) {
+        const nf_sink_plan *const row = s.SinkPlan + (size_t)j * s.Nk;
+        bool bad = false;
+        for (int k = 0; k < s.Nk; k++)
+            for (int c = 1; c < W; c++) {
+                const nf_cell_plan &a = row[k].cell[c], &b = row[k + c < s.cpd ? k + c : k + c - s.cpd].cell[0];
+                bad |= a.start != b.start || a.N != b.N;
             }
-        }
+        if (bad) return fail(NF_ERR_INVALID, "sink plans do not follow the pencil geometry");
+    }
     return NF_OK;
 }
 
@@ -930,7 +1017,7 @@ GPlanScratch gplan_scratch(const std::vector<Task *> &g) {
 // counts from device memory, and the totals come back with the group's
 // results.  Fills in[i] for phase B.
 int plan_phase_a(Runtime &rt, Worker &w, std::vector<Task *> &g, std::vector<Runtime::Slot *> &cslot,
-                 std::vector<GPlanIn> &in, const GPlanScratch &gs, uint64_t *to_dev) {
+                 std::vector<GPlanIn> &in, const GPlanScratch &gs, uint64_t y_cost, uint64_t *to_dev) {
     const size_t n = g.size();
     int rc = w.gscratch.ensure(gs.total);
     if (rc || (rc = w.pin_tot.ensure(256 * n)) || (rc = w.pin_gplan.ensure(gs.total - gs.o_in))) return rc;
@@ -947,7 +1034,9 @@ int plan_phase_a(Runtime &rt, Worker &w, std::vector<Task *> &g, std::vector<Run
         Task &t = *g[i];
         nf_sic &s = t.sic;
         dp_bounds(s, &t.dp.chunks_bound, &t.dp.items_bound);
+        if (y_cost != UINT64_MAX) t.dp.items_bound = y_items_bound(s);
         GPlanIn &gi = in[i];
+        gi.y_cost = y_cost;
         for (int ti = 0; ti < 3; ti++) gi.split_cost[ti] = tile_split_cost(s.softening, 1 << ti, group_est);
         gi.cpd = s.cpd;
         gi.R = s.nfradius;
@@ -998,6 +1087,25 @@ int apply_group_totals(Worker &w, std::vector<Task *> &g) {
     return rc;
 }
 
+// The y_cost of a group's launch: UINT64_MAX (no tile is split over the source
+// pencils, the partials have one plane) unless the launch is small, and its
+// planes and its longer work list fit the buffer.
+uint64_t group_y_cost(const Runtime &rt, const std::vector<Task *> &g) {
+    if (rt.params.path != NF_PATH_BATCHED) return UINT64_MAX;
+    uint64_t work = 0, planes = 0, bytes = 0;
+    for (const Task *t : g) work += queued_interactions(*t);
+    const uint64_t cost = y_split_cost(work, !g[0]->dp.on);
+    if (cost == UINT64_MAX) return cost;
+    for (const Task *t : g) {
+        nf_sic s = t->sic;
+        uint64_t chunks, items;
+        if (t->dp.on) dp_bounds(s, &chunks, &items);
+        planes += y_plane_bytes((uint64_t)s.NSinkBlocks, s.nfwidth);
+        bytes += queued_bytes(*t, rt.params.path) + sizeof(WorkItem) * 3 * y_items_bound(s);  // (3: a trial's lists)
+    }
+    return planes <= kYSplitBytes && bytes + planes <= rt.max_buffer_bytes ? cost : UINT64_MAX;
+}
+
 // Execute a group of compatible SICs on worker w: one plan upload, a gather
 // per SIC, one persistent direct-kernel launch over all their work items
 // (batched path; the plain path launches per SIC), a co-add per SIC.
@@ -1020,11 +1128,12 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     std::vector<Runtime::Slot *> cslot;
     SlotRelease cell_release{rt, cslot};
     uint64_t cell_bytes = 0;
+    const uint64_t y_cost = group_y_cost(rt, g);
     if (dplan) {
         for (Task *t : g)
             if (!t->dp.on) return fail(NF_ERR_STATE, "device-planned and host-planned SICs in one group");
         gs = gplan_scratch(g);
-        const int rc = plan_phase_a(rt, w, g, cslot, gin, gs, &cell_bytes);
+        const int rc = plan_phase_a(rt, w, g, cslot, gin, gs, y_cost, &cell_bytes);
         if (rc) return rc;
         if (path == NF_PATH_BATCHED && rt.autotune)
             for (Task *t : g) dp_occupancy(*t, t->dp.occ);
@@ -1058,22 +1167,22 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     // tiles and of the short tails apart, merged by interleave_pos.
     uint64_t group_total = 0;
     for (int i = 0; i < n; i++) group_total += g[i]->sic.DirectTotal;
-    auto make_items = [&](int S) {
-        std::vector<WorkItem> raw, out;
-        std::vector<uint16_t> bucket;
+    auto make_items = [&](int S, std::vector<WorkItem> &out) {
         const uint64_t max_tile_cost = tile_split_cost(s0.softening, S, group_total);
-        for (int i = 0; i < n; i++) build_items(g[i]->sic, S, i, max_tile_cost, raw, bucket);
-        std::vector<size_t> start(2 * kItemBuckets + 1, 0);
-        for (size_t i = 0; i < raw.size(); i++) start[item_key(raw[i], bucket[i]) + 1]++;
-        for (int b = 0; b < 2 * kItemBuckets; b++) start[b + 1] += start[b];
-        out.resize(raw.size());
-        const int64_t M = (int64_t)start[kItemBuckets], T = (int64_t)raw.size() - M;
-        for (size_t i = 0; i < raw.size(); i++) {
-            const int key = item_key(raw[i], bucket[i]);
-            const int64_t r = (int64_t)start[key]++;
-            out[key < kItemBuckets ? interleave_pos(false, r, M, T) : interleave_pos(true, r - M, M, T)] = raw[i];
+        w.sort_start.assign(2 * kItemBuckets + 1, 0u);
+        w.runs.clear();  // found once: the lookups cost more than the list's own traffic
+        ItemSort sort{w.sort_start.data()};
+        for (int i = 0; i < n; i++) {
+            const nf_sic &s = g[i]->sic;
+            w.nsrc.resize((size_t)s.NSinkSets);
+            for (int k = 0; k < s.NSinkSets; k++) w.nsrc[(size_t)k] = pencil_sources(s, k);
+            for_each_run(s, S, i, max_tile_cost, y_cost, w.nsrc.data(), [&](const ItemRun &r) {
+                sort.add(r);
+                w.runs.push_back(r);
+            });
         }
-        return out;
+        out.resize(sort.begin());
+        for (const ItemRun &r : w.runs) sort.place(r, out.data());
     };
     std::vector<int> Svals;
     if (path == NF_PATH_BATCHED) {
@@ -1084,11 +1193,14 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     }
     // (A device-planned SIC's lists are written on the device; phase A
     // counted their items.)
-    std::vector<std::vector<WorkItem>> itemsets;
+    std::vector<const std::vector<WorkItem> *> itemsets;
     std::vector<size_t> nitems;
     for (int S : Svals) {
-        itemsets.push_back(dplan ? std::vector<WorkItem>() : make_items(S));
-        size_t m = itemsets.back().size();
+        std::vector<WorkItem> &list = w.items[S == 1 ? 0 : S == 2 ? 1 : 2];
+        list.clear();
+        if (!dplan) make_items(S, list);
+        itemsets.push_back(&list);
+        size_t m = list.size();
         if (dplan)
             for (Task *t : g) m += (size_t)t->dp.items_bound;
         nitems.push_back(m);
@@ -1129,7 +1241,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     std::vector<WorkLayout> WL(n);
     size_t work_total = 0;
     for (int i = 0; i < n; i++) {
-        WL[i] = work_layout(g[i]->sic, path, work_total);
+        WL[i] = work_layout(g[i]->sic, path, work_total, y_cost == UINT64_MAX ? 1 : g[i]->sic.nfwidth);
         work_total += WL[i].total;
     }
     // Host mode: every distinct host slab of the group once (through the
@@ -1192,6 +1304,8 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
 
         DevPlan &pl = plans[i];
         pl = dev_plan(s, L, pd);
+        pl.y_cost = y_cost;
+        pl.y_plane = y_cost == UINT64_MAX ? 0 : (int64_t)s.NSinkBlocks * NF_BLOCK_SIZE * 4;
         if (dplan) {  // the actual counts, in device memory; the group's bad cells
             pl.max_src_blocks = g[i]->dp.max_src_blocks;
             char *sc = static_cast<char *>(w.gscratch.p);
@@ -1240,6 +1354,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         v.sources4 = wb + WL[i].o_src;
         v.box4 = box_after(wb + WL[i].o_src, s.NSourceBlocks);
         v.partial = reinterpret_cast<double *>(wb + WL[i].o_part);
+        v.y_plane = pl.y_plane;
         v.W = s.nfwidth;
         v.R = s.nfradius;
     }
@@ -1261,8 +1376,8 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         cfirst[i + 1] = cfirst[i] + group_coadd_waves(plans[i]);
     }
     for (size_t k = 0; k < itemsets.size(); k++)
-        if (!itemsets[k].empty())
-            std::memcpy(hp + o_itemset[k], itemsets[k].data(), sizeof(WorkItem) * itemsets[k].size());
+        if (!itemsets[k]->empty())
+            std::memcpy(hp + o_itemset[k], itemsets[k]->data(), sizeof(WorkItem) * itemsets[k]->size());
     const auto t_fill = clk::now();
     // The plan image goes up on the copy stream, overlapping the kernels of
     // the group before (this worker's previous group has completed, so its
@@ -1471,11 +1586,18 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         if (fresh[k]) upload_ms += event_ms(hslot[k]->t0, hslot[k]->t1);
     if (trial) {
         Runtime::TuneEntry te;
+        // One launch each is a noisy trial (launches of 0.1 ms spread by 15%):
+        // a shape replaces the default only if it is faster by more than that.
         int best = 0;
         for (int c = 0; c < (int)rt.candidates.size(); c++) {
             te.trial_ms.push_back(event_ms(tev[c], tev[c + 1]));
-            if (te.trial_ms[c] < te.trial_ms[best]) best = c;
+            if (rt.candidates[c].sinks_per_lane == rt.shape.sinks_per_lane &&
+                rt.candidates[c].waves_per_wg == rt.shape.waves_per_wg)
+                best = c;
         }
+        const double line = te.trial_ms[best] - std::max(0.02 * te.trial_ms[best], 0.015);
+        for (int c = 0, from = best; c < (int)rt.candidates.size(); c++)
+            if (te.trial_ms[c] < (best == from ? line : te.trial_ms[best])) best = c;
         for (auto &ev : tev) (void)hipEventDestroy(ev);
         te.shape = rt.candidates[best];
         for (Task *t : g) te.interactions += t->sic.DirectTotal;
@@ -1590,6 +1712,12 @@ bool compatible(const nf_sic &a, const nf_sic &b) {
 // gave fuller groups than 1 ms (11.2 launches per step against 12, +0.6%)
 // and 0.5 ms fewer; a uniform box's groups fill at once either way.
 constexpr int kGroupFillWaitUs = 2000;
+// A host-planned group's work list and plan image are built by its worker, in
+// about the time its kernels take, so its SICs are spread over the idle workers
+// once a group holds this many pair interactions (about 1 ms of kernel).  Six
+// SICs of 2e9 went out as groups of 1 and 5, the second 2.6 ms after the first
+// had ended; now as 1, 2, 2 and 1.
+constexpr uint64_t kHostGroupWork = 3000000000ull;
 
 void worker_main(Runtime *rt, Worker *w) {
     for (;;) {
@@ -1606,10 +1734,13 @@ void worker_main(Runtime *rt, Worker *w) {
             if (rt->params.path == NF_PATH_BATCHED && rt->inflight > 0) {
                 const auto deadline = std::chrono::steady_clock::now() + std::chrono::microseconds(kGroupFillWaitUs);
                 auto full = [&] {
-                    if (rt->stopping || rt->queue.empty() || (int)rt->queue.size() >= rt->max_group) return true;
+                    // (nothing in flight any more: the GPU would wait too)
+                    if (rt->stopping || rt->inflight == 0) return true;
+                    if (rt->queue.empty() || (int)rt->queue.size() >= rt->max_group) return true;
                     uint64_t work = 0;
                     for (const Task *t : rt->queue) work += queued_interactions(*t);
-                    return work >= rt->group_interactions;
+                    return work >= (rt->queue.front()->dp.on ? rt->group_interactions
+                                                             : std::min(rt->group_interactions, kHostGroupWork));
                 };
                 while (!full() && rt->qcv.wait_until(lk, deadline) != std::cv_status::timeout) {
                 }
@@ -1625,10 +1756,12 @@ void worker_main(Runtime *rt, Worker *w) {
             // instead of waiting for a whole group to be prepared.
             const int limit = !rt->warm && rt->inflight == 0 ? 1 : rt->max_group;
             rt->warm = true;
+            const size_t idle = std::max<size_t>(1, rt->workers.size() - (size_t)std::max(rt->inflight, 0));
+            const size_t share = (rt->queue.size() + idle) / idle;  // of the SICs waiting, g[0] among them
             rt->inflight++;
             uint64_t work = queued_interactions(*g[0]);
             while (path == NF_PATH_BATCHED && (int)g.size() < limit && work < rt->group_interactions &&
-                   !rt->queue.empty() && rt->queue.front()->dp.on == g[0]->dp.on &&
+                   (g[0]->dp.on || work < kHostGroupWork || g.size() < share) && !rt->queue.empty() && rt->queue.front()->dp.on == g[0]->dp.on &&
                    compatible(g[0]->sic, rt->queue.front()->sic)) {
                 const size_t b = queued_bytes(*rt->queue.front(), path);
                 if (bytes + b > rt->max_buffer_bytes) break;
@@ -1650,6 +1783,7 @@ void worker_main(Runtime *rt, Worker *w) {
             std::lock_guard<std::mutex> lk(rt->qm);
             rt->inflight--;
         }
+        rt->qcv.notify_all();  // (a worker may be waiting for a fuller group)
         for (Task *t : ok) finish(*t, rc);
     }
 }
@@ -1978,6 +2112,7 @@ extern "C" int nf_plan_sic_device(int32_t cpd, int32_t R, int32_t slab, int32_t 
     NF_HIP(hipMalloc(&b.scr, 256 + sizeof(int32_t) * gpu_plan_part_ints(s.NSinkSets, s.NSourceSets)));
     GPlanIn in{};
     for (uint64_t &c : in.split_cost) c = UINT64_MAX;  // (no work lists here)
+    in.y_cost = UINT64_MAX;
     in.cpd = cpd;
     in.R = R;
     in.W = W;
@@ -2224,18 +2359,18 @@ struct NoallocLayout {
     WorkLayout work;
 };
 
-NoallocLayout noalloc_layout(const nf_sic &s) {
+NoallocLayout noalloc_layout(const nf_sic &s, bool y_planes) {
     NoallocLayout L{};
-    // At most one item per padded sink block plus one tail per pencil,
-    // whatever the tile split.
-    L.items_max = (size_t)s.NSinkBlocks + (size_t)s.NSinkSets;
+    // At most one item per padded sink block (and source pencil, if tiles may
+    // be split over them) plus one tail per pencil, whatever the tile split.
+    L.items_max = y_planes ? (size_t)y_items_bound(s) : (size_t)s.NSinkBlocks + (size_t)s.NSinkSets;
     L.o_items = align_up(sizeof(SicView), 256);
     L.o_counter = align_up(L.o_items + sizeof(WorkItem) * std::max<size_t>(L.items_max, 1), 256);
     L.o_plan = align_up(L.o_counter + kCounterBytes, 256);
     L.plan = plan_layout(s, L.o_plan, count_coadd_chunks(s));
     L.image = L.o_plan + L.plan.total;
     L.o_work = align_up(L.image, 256);
-    L.work = work_layout(s, NF_PATH_BATCHED, L.o_work);
+    L.work = work_layout(s, NF_PATH_BATCHED, L.o_work, y_planes ? s.nfwidth : 1);
     L.total = L.o_work + L.work.total;
     return L;
 }
@@ -2266,7 +2401,13 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     if (rc) return rc;
     PairConst pc;
     if ((rc = derive_pair_const(s.softening, s.eps, s.b2, &pc))) return rc;
-    const NoallocLayout L = noalloc_layout(s);
+    // Tiles are split over the source pencils where that fits the scratch too.
+    uint64_t y_cost = y_split_cost(s.DirectTotal, true);
+    NoallocLayout L = noalloc_layout(s, y_cost != UINT64_MAX);
+    if (y_cost != UINT64_MAX && (L.total > NF_NOALLOC_SCRATCH_BYTES || L.image > kNoallocHostBytes)) {
+        y_cost = UINT64_MAX;
+        L = noalloc_layout(s, false);
+    }
     if (L.total > NF_NOALLOC_SCRATCH_BYTES)
         return fail(NF_ERR_CAPACITY, "SIC needs " + std::to_string(L.total) + " bytes of device scratch; "
                                      "nf_execute_sic_noalloc holds " + std::to_string((uint64_t)NF_NOALLOC_SCRATCH_BYTES) +
@@ -2284,7 +2425,9 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
 
     // Plan arrays and the lists derived from them.
     fill_plan_image(s, L.plan, h);
-    const DevPlan pl = dev_plan(s, L.plan, d);
+    DevPlan pl = dev_plan(s, L.plan, d);
+    pl.y_cost = y_cost;
+    pl.y_plane = y_cost == UINT64_MAX ? 0 : (int64_t)s.NSinkBlocks * NF_BLOCK_SIZE * 4;
 
     // The work list, longest items first (items within 1/8 octave of cost
     // keep sink-pencil order), short tails spread through the tiles: a
@@ -2292,20 +2435,12 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     constexpr int S = 2;  // every tile shape gives bitwise the same partials
     const uint64_t split = tile_split_cost(s.softening, S, s.DirectTotal);
     std::fill(g_noalloc_cursor, g_noalloc_cursor + 2 * kItemBuckets + 1, 0u);
-    size_t nitems = 0;
-    for_each_item(s, S, 0, split, [&](const WorkItem &w, uint16_t b) {
-        g_noalloc_cursor[item_key(w, b) + 1]++;
-        nitems++;
-    });
+    ItemSort sort{g_noalloc_cursor};
+    for_each_run(s, S, 0, split, y_cost, nullptr, [&](const ItemRun &r) { sort.add(r); });
+    const size_t nitems = sort.begin();
     if (nitems > L.items_max) return fail(NF_ERR_STATE, "work list longer than its bound");
-    for (int b = 0; b < 2 * kItemBuckets; b++) g_noalloc_cursor[b + 1] += g_noalloc_cursor[b];
-    const int64_t M = g_noalloc_cursor[kItemBuckets], T = (int64_t)nitems - M;
     WorkItem *items = reinterpret_cast<WorkItem *>(h + L.o_items);
-    for_each_item(s, S, 0, split, [&](const WorkItem &w, uint16_t b) {
-        const int key = item_key(w, b);
-        const int64_t r = g_noalloc_cursor[key]++;
-        items[key < kItemBuckets ? interleave_pos(false, r, M, T) : interleave_pos(true, r - M, M, T)] = w;
-    });
+    for_each_run(s, S, 0, split, y_cost, nullptr, [&](const ItemRun &r) { sort.place(r, items); });
 
     DevSlabs sl{};
     for (int c = 0; c < s.nfwidth; c++) {
@@ -2339,6 +2474,7 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     v.sources4 = src;
     v.box4 = box_after(src, s.NSourceBlocks);
     v.partial = reinterpret_cast<double *>(d + L.work.o_part);
+    v.y_plane = pl.y_plane;
     v.W = s.nfwidth;
     v.R = s.nfradius;
 
