@@ -498,80 +498,179 @@ __global__ __launch_bounds__(256) void k_gather_sources_binned_group(const Group
 // Plain path: the reference's structure and pair forms
 // ---------------------------------------------------------------------------
 
-// DirectGPUKernels.cuh direct_density<0>: single spline :68-108, Plummer
-// :144-174, cubic spline :20-66, cubic Plummer :110-143.  rsqrt is the
-// hardware v_rsq_f32 (the reference uses its own platform's fast rsqrtf).
+// What a source tile needs, decided from the tile's bounding box:
+//   kNoDensity  unsoftened branch only, no FOF density (no pair within b)
+//   kDensity    unsoftened branch only, with the FOF density term
+//   kExact      the full softened form with the density term
+// The unsoftened branch equals the full form for every pair with r > e (cubic
+// spline: r > 2 e).
+constexpr int kNoDensity = 0, kDensity = 1, kExact = 2;
+
+// Squared distances above which a form's unsoftened branch is exact and the
+// density term zero.  Both carry a relative margin far above FP32 rounding of
+// the box corners and of r^2.
+struct FormRadii {
+    float soft2, dens2;
+};
+FormRadii form_radii(int softening, const PairConst &pc, float dens_b2) {
+    const double eps = (double)pc.eps;
+    FormRadii f;
+    f.soft2 = softening == NF_SOFT_SINGLE_SPLINE  ? (float)((1.0 / eps) * 1.01)
+              : softening == NF_SOFT_CUBIC_SPLINE ? (float)(4.0 / (eps * eps) * 1.01)
+                                                  : 0.f;
+    f.dens2 = dens_b2 > 0.f ? (float)((double)dens_b2 * 1.01) : -1.f;
+    return f;
+}
+// The form a source tile needs, from the squared gap between its bounding box
+// and the sinks'.
 template <int SOFT>
-__device__ __forceinline__ void ref_pair(float sx, float sy, float sz, float kx, float ky, float kz,
-                                         const PairConst &pc, float &ax, float &ay, float &az, float &aw) {
-    const float dx = sx - kx, dy = sy - ky, dz = sz - kz;
-    const float r2 = dx * dx + dy * dy + dz * dz;
-    if (r2 < pc.b2) aw = aw + pc.b2 - r2;
-    float f;
-    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE) {
-        const float q = r2 * pc.eps + 1e-32f;
-        f = rsq(q);
-        f = (q > 1.0f) ? f * f * f : (-15.0f * f + 6.0f) * q + 10.0f;
-    } else if constexpr (SOFT == NF_SOFT_PLUMMER) {
-        const float r = rsq(r2 + pc.eps);
-        f = r * r * r;
-    } else if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE) {
-        const float rinv = rsq(r2);
-        const float u = pc.eps * sqrt_(r2);  // eps_inv / rinv
-        if (u >= 2.0f) {
-            f = rinv * rinv * rinv;
-        } else if (u >= 1.0f) {
-            const float u3 = u * u * u;
-            f = rinv * rinv * rinv *
-                ((float)(-1.0 / 15.0) + (float)(8.0 / 3.0) * u3 - 3.0f * u3 * u + (float)(6.0 / 5.0) * u3 * u * u -
-                 (float)(1.0 / 6.0) * u3 * u3);
-        } else {
-            f = pc.eps * pc.eps * pc.eps * ((float)(4.0 / 3.0) - (float)(6.0 / 5.0) * u * u + 0.5f * u * u * u);
-        }
-    } else {  // cubic Plummer
-        float r = r2 + 1e-16f;
-        r *= r * rsq(r);
-        r += pc.eps;
-        f = rcp(r);
-    }
-    ax -= f * dx;
-    ay -= f * dy;
-    az -= f * dz;
+__device__ __forceinline__ int form_of(const FormRadii &fr, float gap2) {
+    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE || SOFT == NF_SOFT_CUBIC_SPLINE)
+        if (!(gap2 > fr.soft2)) return kExact;
+    return gap2 <= fr.dens2 ? kDensity : kNoDensity;
 }
 
+// DirectGPUKernels.cuh direct_density<0>: single spline :68-108, Plummer
+// :144-174, cubic spline :20-66, cubic Plummer :110-143.  rsqrt is the
+// hardware v_rsq_f32 (the reference uses its own platform's fast rsqrtf).  The
+// reference's operations in its order; a form leaves out the branches that no
+// pair of its tile takes, so every tile's sums are bitwise the full form's.
+template <int SOFT, int MODE>
+__device__ __forceinline__ void ref_d(float sx, float sy, float sz, float kx, float ky, float kz, const PairConst &pc,
+                                      float &dx, float &dy, float &dz, float &r2, float &aw) {
+    dx = kx - sx, dy = ky - sy, dz = kz - sz;  // (minus the reference's d: a += f d, exactly)
+    r2 = dx * dx + dy * dy + dz * dz;
+    if (MODE != kNoDensity && r2 < pc.b2) aw = aw + pc.b2 - r2;
+}
+// The argument of the form's first transcendental, and f from its value t.
 template <int SOFT>
-__global__ __launch_bounds__(64) void k_plain(DevPlan pl, PairConst pc, const float4 *__restrict__ sinks,
-                                              const float4 *__restrict__ src, float4 *__restrict__ out) {
+__device__ __forceinline__ float ref_arg(float r2, const PairConst &pc) {
+    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE) return r2 * pc.eps + 1e-32f;
+    else if constexpr (SOFT == NF_SOFT_PLUMMER) return r2 + pc.eps;
+    else if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE) return r2;
+    else return r2 + 1e-16f;
+}
+template <int SOFT, int MODE>
+__device__ __forceinline__ float ref_f(float q, float t, const PairConst &pc) {
+    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE) {
+        const float f3 = t * t * t;
+        if constexpr (MODE != kExact) return f3;
+        return (q > 1.0f) ? f3 : (-15.0f * t + 6.0f) * q + 10.0f;
+    } else if constexpr (SOFT == NF_SOFT_PLUMMER) {
+        return t * t * t;
+    } else if constexpr (SOFT == NF_SOFT_CUBIC_SPLINE) {
+        const float f3 = t * t * t;
+        if constexpr (MODE != kExact) return f3;
+        const float u = pc.eps * sqrt_(q);  // eps_inv / rinv
+        if (u >= 2.0f) return f3;
+        if (u >= 1.0f) {
+            const float u3 = u * u * u;
+            return f3 * ((float)(-1.0 / 15.0) + (float)(8.0 / 3.0) * u3 - 3.0f * u3 * u +
+                         (float)(6.0 / 5.0) * u3 * u * u - (float)(1.0 / 6.0) * u3 * u3);
+        }
+        return pc.eps * pc.eps * pc.eps * ((float)(4.0 / 3.0) - (float)(6.0 / 5.0) * u * u + 0.5f * u * u * u);
+    } else {  // cubic Plummer
+        float r = q;
+        r *= r * t;
+        r += pc.eps;
+        return rcp(r);
+    }
+}
+// P sources against the lane's sink, in order.
+template <int SOFT, int MODE, int P>
+__device__ __forceinline__ void ref_pairs(const NF_CONST float4 *sp, float yo, float4 k, const PairConst &pc,
+                                          float &ax, float &ay, float &az, float &aw) {
+    float dx[P], dy[P], dz[P], q[P], t[P];
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        const float4 s = sp[i];
+        float r2;
+        ref_d<SOFT, MODE>(s.x, s.y + yo, s.z, k.x, k.y, k.z, pc, dx[i], dy[i], dz[i], r2, aw);
+        t[i] = q[i] = ref_arg<SOFT>(r2, pc);
+    }
+    if constexpr (P == 1) NF_TRANS1("v_rsq_f32", t[0]);
+#pragma unroll
+    for (int i = 0; i + 1 < P; i += 2) NF_TRANS2("v_rsq_f32", t[i], t[i + 1]);
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        const float f = ref_f<SOFT, MODE>(q[i], t[i], pc);
+        ax += f * dx[i];
+        ay += f * dy[i];
+        az += f * dz[i];
+    }
+}
+// A tile of 64 sources (FullDirectTile with BLOCK_ACCUM), or the first cnt of
+// one (PartialDirectTile, straight into the sink's sums).
+template <int SOFT, int MODE>
+__device__ __forceinline__ void ref_tile(const NF_CONST float4 *sp, int cnt, float yo, float4 k, const PairConst &pc,
+                                         float &ax, float &ay, float &az, float &aw) {
+    if (cnt == kWave) {
+        float tx = 0.f, ty = 0.f, tz = 0.f;
+        for (int i = 0; i < kWave; i += 16)
+#pragma unroll
+            for (int q = 0; q < 16; q += 2) ref_pairs<SOFT, MODE, 2>(sp + i + q, yo, k, pc, tx, ty, tz, aw);
+        ax += tx;
+        ay += ty;
+        az += tz;
+        return;
+    }
+    int i = 0;
+    for (; i + 4 <= cnt; i += 4) {
+        ref_pairs<SOFT, MODE, 2>(sp + i, yo, k, pc, ax, ay, az, aw);
+        ref_pairs<SOFT, MODE, 2>(sp + i + 2, yo, k, pc, ax, ay, az, aw);
+    }
+    for (; i < cnt; i++) ref_pairs<SOFT, MODE, 1>(sp + i, yo, k, pc, ax, ay, az, aw);
+}
+
+// One 64-sink block per wave, every source pencil in turn.  VALU-bound: the
+// full form of the single spline is 21 VALU instructions and a v_rsq_f32 per
+// pair, of which the unsoftened form without the density needs 13; 78% of a
+// uniform box's tiles take that one.  Eight slabs of a uniform 256^3 box: 7.95 ms as one loop of
+// full forms, 5.89 with the v_rsq at raised priority, 4.55 with the forms.
+template <int SOFT>
+__global__ __launch_bounds__(64) void k_plain(DevPlan pl, PairConst pc, FormRadii fr,
+                                              const float4 *__restrict__ sinks, const float4 *__restrict__ src,
+                                              float4 *__restrict__ out) {
     const int blk = blockIdx.x;
     if (blk >= sink_blocks(pl) || plan_bad(pl)) return;
-    const int s = pl.parent[blk];
-    const int id = blk * kWave + threadIdx.x;
+    const int lane = threadIdx.x;
+    const int s = cptr<int32_t>(pl.parent)[blk];
+    const int id = blk * kWave + lane;
     const float4 k = sinks[id];  // padded ids hold zeros (PencilKernel.cu:109-117)
+    const bool real = (uint32_t)id < cptr<uint32_t>(pl.sink_idmax)[s];
+    const float inf = __builtin_huge_valf();
+    const float lx = wave_min(real ? k.x : inf), ly = wave_min(real ? k.y : inf), lz = wave_min(real ? k.z : inf);
+    const float hx = wave_max(real ? k.x : -inf), hy = wave_max(real ? k.y : -inf), hz = wave_max(real ? k.z : -inf);
+    const NF_CONST float4 *sources = cptr<float4>(src);
+    const NF_CONST float4 *box = sources + (int64_t)pl.nsrc_blocks * kWave;  // box_after
     float ax = 0.f, ay = 0.f, az = 0.f, aw = 0.f;
     const int W = pl.W;
     for (int c = s * W; c < s * W + W; c++) {
-        const int si = pl.ilist[c];
-        const float yo = pl.yoff[c];
-        const int st = pl.src_set_start[si], n = pl.src_set_count[si];
-        const float4 *sp = src + st;
-        const int nB = n / kWave;
-        for (int b = 0; b < nB; b++) {  // FullDirectTile with BLOCK_ACCUM
-            float tx = 0.f, ty = 0.f, tz = 0.f;
-#pragma unroll 16
-            for (int i = 0; i < kWave; i++) {
-                const float4 q = sp[b * kWave + i];
-                ref_pair<SOFT>(q.x, q.y + yo, q.z, k.x, k.y, k.z, pc, tx, ty, tz, aw);
+        const int si = cptr<int32_t>(pl.ilist)[c];
+        const float yo = cptr<float>(pl.yoff)[c];
+        const int st = cptr<int32_t>(pl.src_set_start)[si], n = cptr<int32_t>(pl.src_set_count)[si];
+        int forms = 0;  // lane i: the form of tile (b & ~63) + i
+        for (int b = 0; b * kWave < n; b++) {
+            if ((b & (kWave - 1)) == 0) {
+                forms = 0;
+                if ((b + lane) * kWave < n) {
+                    const int64_t gb = (int64_t)st / kWave + b + lane;
+                    const float4 ql = box[2 * gb], qh = box[2 * gb + 1];
+                    const float gx = fmaxf(0.f, fmaxf(ql.x - hx, lx - qh.x));
+                    const float gy = fmaxf(0.f, fmaxf(ql.y + yo - hy, ly - (qh.y + yo)));
+                    const float gz = fmaxf(0.f, fmaxf(ql.z - hz, lz - qh.z));
+                    forms = form_of<SOFT>(fr, gx * gx + gy * gy + gz * gz);
+                }
             }
-            ax += tx;
-            ay += ty;
-            az += tz;
-        }
-        for (int i = nB * kWave; i < n; i++) {  // PartialDirectTile
-            const float4 q = sp[i];
-            ref_pair<SOFT>(q.x, q.y + yo, q.z, k.x, k.y, k.z, pc, ax, ay, az, aw);
+            const int form = __builtin_amdgcn_readlane(forms, b & (kWave - 1));
+            const NF_CONST float4 *sp = sources + st + b * kWave;
+            const int cnt = min(kWave, n - b * kWave);
+            if (form == kNoDensity) ref_tile<SOFT, kNoDensity>(sp, cnt, yo, k, pc, ax, ay, az, aw);
+            else if (form == kDensity) ref_tile<SOFT, kDensity>(sp, cnt, yo, k, pc, ax, ay, az, aw);
+            else ref_tile<SOFT, kExact>(sp, cnt, yo, k, pc, ax, ay, az, aw);
         }
     }
-    if ((uint32_t)id < pl.sink_idmax[s]) out[id] = make_float4(ax, ay, az, aw);
+    if (real) out[id] = make_float4(ax, ay, az, aw);
 }
 
 // Addresses of the W partials of the sinks of cell (j_low + j, z): the cell is
@@ -713,13 +812,8 @@ __global__ __launch_bounds__(256) void k_coadd_f64_group(const GroupSic *__restr
 // ---------------------------------------------------------------------------
 
 // Pair kernel in box units.  r2 carries pc.r2add; for the single spline the
-// result is g/e^3 (the e^3 is restored in the co-add).  MODE selects what a
-// source tile needs, decided from the tile's bounding box:
-//   kNoDensity  unsoftened branch only, no FOF density (no pair within b)
-//   kDensity    unsoftened branch only, with the FOF density term
-//   kExact      the full softened form with the density term
-// The unsoftened branch equals the full form for every pair with r > e.
-constexpr int kNoDensity = 0, kDensity = 1, kExact = 2;
+// result is g/e^3 (the e^3 is restored in the co-add).  MODE: the tile's form,
+// as on the plain path.
 
 // A pair in four steps, so that the transcendentals of two pairs can run in
 // one raised stretch (35.9 -> 35.4 cycles per pair):
@@ -823,8 +917,7 @@ __device__ __forceinline__ void pair_group(const NF_CONST float4 *sp, const floa
 struct BatchCtx {
     PairConst pc;
     double invcpd;
-    float soft2;  // squared distance above which the unsoftened branch is exact (with margin)
-    float dens2;  // squared distance above which the FOF density term is zero (with margin)
+    FormRadii fr;
 };
 
 // A sink pencil's cells, for reading its sinks straight from the slab.
@@ -859,15 +952,6 @@ __device__ __forceinline__ float3 pencil_sink(const SicView &v, const SinkCells 
     }
     const float3 q = slab_xyz(v.sink_slab, v.sink_n, (uint64_t)start + (uint64_t)(i - pre), v.aos);
     return make_float3(q.x, q.y, (float)((double)q.z + (double)(c - v.R) * invcpd));
-}
-
-// The mode a source tile needs, from the squared gap between its bounding box
-// and the sinks' bounding box (wave-uniform).
-template <int SOFT>
-__device__ __forceinline__ int tile_mode(const BatchCtx &cx, float gap2) {
-    if constexpr (SOFT == NF_SOFT_SINGLE_SPLINE || SOFT == NF_SOFT_CUBIC_SPLINE)
-        if (!cx.pc.fast_ok || gap2 <= cx.soft2) return kExact;
-    return gap2 <= cx.dens2 ? kDensity : kNoDensity;
 }
 
 // A sink pencil's W source pencils: lane y holds pencil y's first slot and
@@ -921,11 +1005,11 @@ __device__ __forceinline__ int block_forms(const BatchCtx &cx, const SicView &v,
     const float gy = fmaxf(0.f, fmaxf(ql.y - shy, sly - qh.y));
     const float gxy = gx * gx + gy * gy;
     const float gz1 = fmaxf(0.f, fmaxf(ql.z - k.hz1, k.lz1 - qh.z));
-    const int mh = tile_mode<SOFT>(cx, gxy + gz1 * gz1);
+    const int mh = form_of<SOFT>(cx.fr, gxy + gz1 * gz1);
     int ml = mh;
     if (HALVES) {
         const float gz0 = fmaxf(0.f, fmaxf(ql.z - k.hz0, k.lz0 - qh.z));
-        ml = tile_mode<SOFT>(cx, gxy + gz0 * gz0);
+        ml = form_of<SOFT>(cx.fr, gxy + gz0 * gz0);
     }
     return ml | (mh << 2);
 }
@@ -1455,7 +1539,7 @@ template <int SOFT>
 int launch_plain_t(const DevPlan &pl, const PairConst &pc, const void *sinks4, const void *sources4, void *partial4,
                    hipStream_t st) {
     if (pl.nsink_blocks == 0) return 0;
-    hipLaunchKernelGGL(k_plain<SOFT>, dim3(pl.nsink_blocks), dim3(kWave), 0, st, pl, pc,
+    hipLaunchKernelGGL(k_plain<SOFT>, dim3(pl.nsink_blocks), dim3(kWave), 0, st, pl, pc, form_radii(SOFT, pc, pc.b2),
                        static_cast<const float4 *>(sinks4), static_cast<const float4 *>(sources4),
                        static_cast<float4 *>(partial4));
     return (int)hipGetLastError();
@@ -1624,15 +1708,7 @@ int launch_batched(const SicView *views, int cpd, int softening, const PairConst
     BatchCtx cx;
     cx.pc = pc;
     cx.invcpd = 1.0 / (double)cpd;
-    // The unsoftened branch is exact for r^2 > e^2 = 1/eps (single spline) and
-    // for r > 2 e = 2/eps (cubic spline); the box test uses a relative margin
-    // far above FP32 rounding of the box corners.
-    cx.soft2 = softening == NF_SOFT_SINGLE_SPLINE  ? (float)((1.0 / (double)pc.eps) * 1.01)
-               : softening == NF_SOFT_CUBIC_SPLINE ? (float)(4.0 / ((double)pc.eps * (double)pc.eps) * 1.01)
-                                                   : 0.f;
-    // Density is nonzero only for r^2 + r2add < b2x; a 1% margin covers the
-    // FP32 rounding of the box gap and of r^2.
-    cx.dens2 = pc.b2x > 0.f ? (float)((double)pc.b2x * 1.01) : -1.f;
+    cx.fr = form_radii(softening, pc, pc.b2x);  // (density is nonzero only for r^2 + r2add < b2x)
     switch (softening) {
         case NF_SOFT_PLUMMER: return launch_batched_soft<NF_SOFT_PLUMMER>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
         case NF_SOFT_SINGLE_SPLINE:

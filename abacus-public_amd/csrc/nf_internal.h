@@ -150,7 +150,6 @@ struct PairConst {
     float c1, c2, c3; // single spline, box-unit polynomial (-15 e^-4, 6 e^-5, 10 e^-3); cubic spline: c3 = e^-3
     float theta;      // tile density sum below which no pair is softened (< 0: none)
     double out_scale; // e^3 for the box-unit spline, 1 otherwise
-    int32_t fast_ok;  // 1 when the unsoftened fast path may be used
 };
 
 int derive_pair_const(int softening, float eps, float b2, PairConst *pc);

@@ -67,14 +67,12 @@ int derive_pair_const(int softening, float eps, float b2, PairConst *pc) {
             pc->out_scale = 1.0 / (e * std::sqrt(e));
             if (!std::isfinite(pc->c1) || !std::isfinite(pc->c2) || !std::isfinite(pc->c3) || pc->c1 == 0.f)
                 return fail(NF_ERR_INVALID, "single spline eps out of the FP32 box-unit range");
-            pc->fast_ok = 1;
             break;
         }
         case NF_SOFT_PLUMMER: pc->r2add = eps; break;
         case NF_SOFT_CUBIC_SPLINE:
             pc->r2add = 1e-24f;  // as the single spline's: keeps the self pair's 1/r finite
             pc->c3 = eps * eps * eps;
-            pc->fast_ok = 1;
             break;
         case NF_SOFT_CUBIC_PLUMMER: pc->r2add = 1e-16f; break;  // TAU2, DirectGPUKernels.cuh:113
         default: return fail(NF_ERR_INVALID, "unknown softening");

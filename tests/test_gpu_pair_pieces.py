@@ -51,3 +51,25 @@ def test_pair_pieces_vs_fp64(softening):
             tol = 4 * 3 * 0.36 * 2.0 ** -25 / (0.3 * 0.004) + 10 * 2.0 ** -24
             assert rel_err(acc, ref).max() <= tol
             assert np.abs(acc[:, 3] - ref[:, 3]).max() <= 1e-5 * float(b2) * len(U)
+
+
+@pytest.mark.parametrize("softening", sorted(synth.SOFTENINGS))
+def test_plain_pair_pieces_vs_fp64(softening):
+    """The same on the plain path, whose tiles leave out branches by their boxes."""
+    box, soft, e = _pairs_box(softening)
+    eps, _ = synth.eps_param(softening, soft)
+    b2 = synth.fof_b2(2.5 * e / 0.25)
+    with nfm.NearFieldDriver(box.cpd, soft, b2, softening=softening, path="plain", buffers_per_device=1,
+                             max_buffer_bytes=1 << 30) as drv:
+        for x in (3, 4):
+            n = box.slab(x).n
+            acc = np.full((n, 4), np.nan, np.float32)
+            drv.execute_slab(box, x, acc, blocking=True)
+            drv.finalize(x)
+            sl, ix, ce = po.slab_sinks(box, x)
+            ref = po.direct_f64(box, R, softening, eps, b2, sl, ix, ce)
+            # as above, with the FLOAT cell offsets' rounding in each coordinate too; the cubic
+            # spline's middle piece cancels to a 50th of its terms near r = 2 e
+            tol = 2 * 4 * 3 * 0.36 * 2.0 ** -25 / (0.3 * 0.004) + 10 * 50 * 2.0 ** -24
+            assert rel_err(acc, ref).max() <= tol
+            assert np.abs(acc[:, 3] - ref[:, 3]).max() <= 1e-5 * float(b2) * len(U)
