@@ -23,6 +23,7 @@
 //       offsets from an in-LDS scan of the histogram).
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 #include "nf_internal.h"
@@ -34,23 +35,27 @@ constexpr int kB = NF_BLOCK_SIZE;
 constexpr int kT = 256;  // threads per workgroup of the planner kernels
 static_assert(kPlanBuckets == 2 * kT, "k_plan_b2 scans the histogram two buckets per thread");
 
+// A SIC's inputs or outputs of a group launch, by scalar loads (the workgroup's
+// SIC is wave-uniform).
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const __attribute__((address_space(4))) T *)p;
+#else
+    return *p;
+#endif
+}
+
 __device__ __forceinline__ int wrapi(int i, int n) { return i >= n ? i - n : (i < 0 ? i + n : i); }
 __device__ __forceinline__ int nblocks(int n) { return (n + kB - 1) / kB; }
 __host__ __device__ inline int ngroups(int n) { return (n + kT - 1) / kT; }
 
-// Sum over the wave, then one atomic per wave.
-__device__ __forceinline__ void wave_add(uint64_t *p, uint64_t v) {
+__device__ __forceinline__ uint64_t wave_sum(uint64_t v) {
     for (int off = 32; off >= 1; off >>= 1) {
         const uint32_t lo = __shfl_xor((uint32_t)v, off), hi = __shfl_xor((uint32_t)(v >> 32), off);
         v += ((uint64_t)hi << 32) | lo;
     }
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd((unsigned long long *)p, (unsigned long long)v);
-}
-
-// The same for a 32-bit counter.
-__device__ __forceinline__ void wave_add32(int32_t *p, int32_t v) {
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(p, v);
+    return v;
 }
 
 // Whether a planned cell (start as the plan stores it) lies inside its slab.
@@ -67,16 +72,28 @@ __device__ __forceinline__ const nf_cellinfo *sink_row(const GPlanIn &in, int j)
 __device__ __forceinline__ int source_cell(const GPlanIn &in, int jj, int k) {
     return wrapi(jj + in.j_low - in.R, in.cpd) * in.cpd + wrapi(k + in.R, in.cpd);
 }
+// (The loops over the width run to the largest one, past W on the last slab or
+// row again: unrolled, their loads are in flight together.  As loops of W they
+// waited for one load after the other, 25 of them per pencil, which was most of
+// the planning kernels' 10 to 40 us.)
 __device__ __forceinline__ int source_pencil_count(const GPlanIn &in, int jj, int k) {
     const int cell = source_cell(in, jj, k);
     int n = 0;
-    for (int c = 0; c < in.W; c++) n += in.ci[c][cell].count;
+#pragma unroll
+    for (int c = 0; c < NF_MAX_WIDTH; c++) {
+        const int m = in.ci[c < in.W ? c : 0][cell].count;
+        n += c < in.W ? m : 0;
+    }
     return n;
 }
 // Sources sink pencil (j, k) meets: its W source pencils (j + y, k).
 __device__ __forceinline__ uint64_t sink_pencil_sources(const GPlanIn &in, int j, int k) {
     uint64_t n = 0;
-    for (int y = 0; y < in.W; y++) n += (uint64_t)source_pencil_count(in, j + y, k);
+#pragma unroll
+    for (int y = 0; y < NF_MAX_WIDTH; y++) {
+        const int m = source_pencil_count(in, j + (y < in.W ? y : 0), k);
+        n += y < in.W ? (uint64_t)m : 0;
+    }
     return n;
 }
 
@@ -167,10 +184,13 @@ __device__ void plan_a(const GPlanIn &in, GPlanTotals *tot, int32_t *group, int 
         const int j = t / in.cpd, k = t % in.cpd;
         const nf_cellinfo *row = sink_row(in, j);
         int n = 0;
-        for (int c = 0; c < in.W; c++) {
-            const nf_cellinfo &ci = row[wrapi(k + c, in.cpd)];
-            n += ci.count;
-            bad += cell_ok(ci.startindex, ci.count, in.nslab[in.R]) ? 0 : 1;
+#pragma unroll
+        for (int c = 0; c < NF_MAX_WIDTH; c++) {
+            const nf_cellinfo &ci = row[wrapi(k + (c < in.W ? c : 0), in.cpd)];
+            const int m = ci.count;
+            const uint64_t start = ci.startindex;
+            n += c < in.W ? m : 0;
+            bad += c < in.W && !cell_ok(start, m, in.nslab[in.R]) ? 1 : 0;
         }
         sink = (uint64_t)n;
         sblk = (uint64_t)nblocks(n);
@@ -185,27 +205,49 @@ __device__ void plan_a(const GPlanIn &in, GPlanTotals *tot, int32_t *group, int 
         const int u = t - P;
         const int cell = source_cell(in, u / in.cpd, u % in.cpd);
         int n = 0;
-        for (int c = 0; c < in.W; c++) {
-            const nf_cellinfo &ci = in.ci[c][cell];
-            n += ci.count;
-            bad += cell_ok(ci.startindex_with_ghost, ci.count, in.nslab[c]) ? 0 : 1;
+#pragma unroll
+        for (int c = 0; c < NF_MAX_WIDTH; c++) {
+            const nf_cellinfo &ci = in.ci[c < in.W ? c : 0][cell];
+            const int m = ci.count;
+            const uint64_t start = ci.startindex_with_ghost;
+            n += c < in.W ? m : 0;
+            bad += c < in.W && !cell_ok(start, m, in.nslab[c < in.W ? c : 0]) ? 1 : 0;
         }
         src = (uint64_t)n;
         qblk = (uint64_t)nblocks(n);
     }
-    wave_add(&tot->sink_total, sink);
-    wave_add(&tot->sink_blocks, sblk);
-    wave_add(&tot->chunks, ch);
-    for (int i = 0; i < 3; i++) wave_add(&tot->items[i], it[i]);
-    for (int i = 0; i < 4; i++) wave_add(&tot->occ[i], occ[i]);
-    wave_add(&tot->source_total, src);
-    wave_add(&tot->source_blocks, qblk);
-    wave_add(&tot->bad, bad);
-    wave_add(&tot->direct_total, d);
-    wave_add(&tot->padded_direct_total, pd);
-    if (group) {
-        for (int i = 0; i < 3; i++) wave_add32(group + kPlanGroupItems + i, (int32_t)it[i]);
-        wave_add32(group + kPlanGroupBad, bad ? 1 : 0);  // pencils with a bad cell
+    // Sums over the workgroup in LDS, then one atomic instruction for all the
+    // totals: atomics on one address retire one per 11.7 ns, and one per wave
+    // and total took 20-25 us of a 129^2-cell SIC.
+    constexpr int kTotals = sizeof(GPlanTotals) / sizeof(uint64_t);
+    __shared__ unsigned long long sums[kTotals];
+    if (threadIdx.x < kTotals) sums[threadIdx.x] = 0;
+    __syncthreads();
+    auto add = [&](size_t byte, uint64_t v) {
+        v = wave_sum(v);
+        if ((threadIdx.x & 63) == 0 && v) atomicAdd(&sums[byte / sizeof(uint64_t)], (unsigned long long)v);
+    };
+    if (bid * kT < P) {  // a workgroup with sink pencils
+        add(offsetof(GPlanTotals, sink_total), sink);
+        add(offsetof(GPlanTotals, sink_blocks), sblk);
+        add(offsetof(GPlanTotals, chunks), ch);
+        for (int i = 0; i < 3; i++) add(offsetof(GPlanTotals, items) + 8 * i, it[i]);
+        for (int i = 0; i < 4; i++) add(offsetof(GPlanTotals, occ) + 8 * i, occ[i]);
+        add(offsetof(GPlanTotals, direct_total), d);
+        add(offsetof(GPlanTotals, padded_direct_total), pd);
+    }
+    if (bid * kT + kT > P) {  // with source pencils
+        add(offsetof(GPlanTotals, source_total), src);
+        add(offsetof(GPlanTotals, source_blocks), qblk);
+    }
+    add(offsetof(GPlanTotals, bad), bad);
+    __syncthreads();
+    if (threadIdx.x < kTotals && sums[threadIdx.x])
+        atomicAdd(reinterpret_cast<unsigned long long *>(tot) + threadIdx.x, sums[threadIdx.x]);
+    if (group && threadIdx.x < 4) {  // work items per tile, bad cells
+        static_assert(kPlanGroupBad == kPlanGroupItems + 3, "the bad cells follow the items");
+        const size_t f = threadIdx.x < 3 ? offsetof(GPlanTotals, items) / 8 + threadIdx.x : offsetof(GPlanTotals, bad) / 8;
+        if (sums[f]) atomicAdd(group + kPlanGroupItems + threadIdx.x, (int32_t)sums[f]);
     }
 }
 __global__ __launch_bounds__(kT) void k_plan_a(GPlanIn in, GPlanTotals *tot, int32_t *group) {
@@ -233,16 +275,14 @@ __device__ void plan_b1(const GPlanIn &in, const GPlanOut &out, int bid) {
             const nf_cellinfo *row = sink_row(in, j);
             nf_sink_plan pl;
             int n = 0;
+#pragma unroll
             for (int c = 0; c < NF_MAX_WIDTH; c++) {
-                if (c < in.W) {
-                    const nf_cellinfo &ci = row[wrapi(k + c, in.cpd)];
-                    pl.cell[c].start = (uint32_t)ci.startindex;
-                    pl.cell[c].N = ci.count;
-                    n += ci.count;
-                } else {
-                    pl.cell[c].start = 0;
-                    pl.cell[c].N = 0;
-                }
+                const nf_cellinfo &ci = row[wrapi(k + (c < in.W ? c : 0), in.cpd)];
+                const uint32_t start = (uint32_t)ci.startindex;
+                const int32_t m = ci.count;
+                pl.cell[c].start = c < in.W ? start : 0;
+                pl.cell[c].N = c < in.W ? m : 0;
+                n += pl.cell[c].N;
             }
             // The cell that sits at z = 0 after the periodic wrap
             // (PencilPlan.cc:123-128): k + c = cpd, if within the pencil.
@@ -281,16 +321,14 @@ __device__ void plan_b1(const GPlanIn &in, const GPlanOut &out, int bid) {
             const int cell = source_cell(in, u / in.cpd, u % in.cpd);
             nf_source_plan pl;
             int n = 0;
+#pragma unroll
             for (int c = 0; c < NF_MAX_WIDTH; c++) {
-                if (c < in.W) {
-                    const nf_cellinfo &ci = in.ci[c][cell];
-                    pl.cell[c].start = (uint32_t)ci.startindex_with_ghost;
-                    pl.cell[c].N = ci.count;
-                    n += ci.count;
-                } else {
-                    pl.cell[c].start = 0;
-                    pl.cell[c].N = 0;
-                }
+                const nf_cellinfo &ci = in.ci[c < in.W ? c : 0][cell];
+                const uint32_t start = (uint32_t)ci.startindex_with_ghost;
+                const int32_t m = ci.count;
+                pl.cell[c].start = c < in.W ? start : 0;
+                pl.cell[c].N = c < in.W ? m : 0;
+                n += pl.cell[c].N;
             }
             out.src_plan[u] = pl;
             out.src_count[u] = n;
@@ -449,17 +487,17 @@ __global__ void k_plan_zero_group(char *tot, int n, int32_t *shared, int nshared
 __global__ __launch_bounds__(kT) void k_plan_a_group(const GPlanIn *__restrict__ ins, char *tot, int32_t *group,
                                                      const int32_t *__restrict__ first, int n) {
     const int s = group_sic(first, n, (int)blockIdx.x);
-    plan_a(ins[s], reinterpret_cast<GPlanTotals *>(tot + 256 * (size_t)s), group, (int)blockIdx.x - first[s]);
+    plan_a(uniform_load(ins + s), reinterpret_cast<GPlanTotals *>(tot + 256 * (size_t)s), group, (int)blockIdx.x - first[s]);
 }
 __global__ __launch_bounds__(kT) void k_plan_b1_group(const GPlanIn *__restrict__ ins, const GPlanOut *__restrict__ outs,
                                                       const int32_t *__restrict__ first, int n) {
     const int s = group_sic(first, n, (int)blockIdx.x);
-    plan_b1(ins[s], outs[s], (int)blockIdx.x - first[s]);
+    plan_b1(uniform_load(ins + s), uniform_load(outs + s), (int)blockIdx.x - first[s]);
 }
 __global__ __launch_bounds__(kT) void k_plan_b2_group(const GPlanIn *__restrict__ ins, const GPlanOut *__restrict__ outs,
                                                       const int32_t *__restrict__ first, int n) {
     const int s = group_sic(first, n, (int)blockIdx.x);
-    plan_b2(ins[s], outs[s], (int)blockIdx.x - first[s]);
+    plan_b2(uniform_load(ins + s), uniform_load(outs + s), (int)blockIdx.x - first[s]);
 }
 
 }  // namespace

@@ -323,6 +323,53 @@ struct BlockBox {
     }
 };
 
+// A pencil of at most one block (total <= 64 sources): a source to a lane, all
+// cells at once.  A lane's rank among its cell's lanes comes from the same 8
+// ballots, cut down to the cell: 100 instructions instead of 5 x 70 and one
+// load instead of one after the other per cell.  A launch group of sparse SICs
+// (129^2 pencils of 25 sources each): 105 -> 52 us on average.
+__device__ __forceinline__ void gather_small_pencil(const DevPlan &pl, const DevSlabs &sl, const nf_source_plan &p,
+                                                    const int *pre, int total, float4 *__restrict__ dst,
+                                                    float4 *__restrict__ box, float cpdf, double invcpd, int lane) {
+    int c = 0, first = 0, next = pre[1];
+    uint32_t start = p.cell[0].start;
+    const float *P = sl.pos[0];
+    uint64_t ns = sl.n[0];
+#pragma unroll
+    for (int k = 1; k < NF_MAX_WIDTH; k++) {
+        const bool in = lane >= pre[k] && pre[k + 1] > pre[k];
+        c = in ? k : c;
+        first = in ? pre[k] : first;
+        next = in ? pre[k + 1] : next;
+        start = in ? p.cell[k].start : start;
+        P = in ? sl.pos[k] : P;
+        ns = in ? sl.n[k] : ns;
+    }
+    const bool live = lane < total;
+    const float3 q = live ? slab_xyz(P, ns, (uint64_t)start + (uint64_t)(lane - first), sl.aos)
+                          : make_float3(0.f, 0.f, 0.f);
+    const int bin = live ? xbin(q.x, cpdf) : -1;
+    const int n = next - first;
+    const uint64_t cell = (n >= kWave ? ~0ull : (1ull << n) - 1) << first;
+    const uint64_t below = cell & ((1ull << lane) - 1);
+    int rank = 0;
+#pragma unroll
+    for (int k = 0; k < kXBins; k++) {
+        const uint64_t m = ballot(bin == k);
+        rank += __builtin_popcountll(m & (k < bin ? cell : k == bin ? below : 0ull));
+    }
+    const float x = (float)((double)q.x + (double)(c - pl.R) * invcpd);
+    dst[live ? first + rank : lane] = live ? make_float4(x, q.y, q.z, 0.f) : make_float4(kFar, 0.f, 0.f, 0.f);
+    const float inf = __builtin_huge_valf();
+    const float4 lo = make_float4(wave_min(live ? x : inf), wave_min(live ? q.y : inf), wave_min(live ? q.z : inf), 0.f);
+    const float4 hi =
+        make_float4(wave_max(live ? x : -inf), wave_max(live ? q.y : -inf), wave_max(live ? q.z : -inf), 0.f);
+    if (lane == 0) {
+        box[0] = lo;
+        box[1] = hi;
+    }
+}
+
 // Blocks [blo, bhi) of pencil s (pencil-relative; bhi may pass its end);
 // RANGED false: the whole pencil, without the range tests.
 template <bool RANGED>
@@ -342,6 +389,10 @@ __device__ __forceinline__ void gather_pencil_binned(const DevPlan &pl, const De
     const int start = cptr<int32_t>(pl.src_set_start)[s];  // the pencil's first slot, a multiple of 64
     float4 *dst = out + start;
     const int64_t gb0 = start / kWave;
+    if (total <= kWave) {  // (its range is the whole pencil)
+        gather_small_pencil(pl, sl, p, pre, total, dst, box + 2 * gb0, cpdf, invcpd, lane);
+        return;
+    }
     const int last = (total - 1) / kWave;
     if ((!RANGED || (last >= blo && last < bhi)) && last * kWave + lane >= total)
         dst[last * kWave + lane] = make_float4(kFar, 0.f, 0.f, 0.f);
@@ -453,10 +504,28 @@ __device__ __forceinline__ void gather_wave(const DevPlan &pl, const DevSlabs &s
     if (lo < hi) gather_pencil_binned<true>(pl, sl, out, box, cpdf, invcpd, s, lane, lo - f, hi - f);
 }
 
+// Clears the batched launch's queues and, for a census build, its census; for a
+// device-planned list, copies its length into counter[1], or 0 when the group
+// holds a cell outside its slab.  The first workgroup of the gather does it
+// (a launch of its own took 4 us, and a gap), or k_zero_counter.
+constexpr int kCensusOffset = kCensusBytes / 4;  // int32 units
+constexpr int kQueueOffset = kQueueBytes / 4, kQueueStride = kQueueLine / 4;
+__device__ __forceinline__ void clear_queues(const QueueClear &qc, int t) {
+    int32_t *const c = qc.counter;
+    if (t < kQueues) c[kQueueOffset + t * kQueueStride] = 0;
+    if (t != 0) return;
+    if (qc.dnitems) c[1] = (qc.dbad && *qc.dbad != 0) ? 0 : *qc.dnitems;
+    if (qc.census) {
+        unsigned long long *cs = reinterpret_cast<unsigned long long *>(c + kCensusOffset);
+        for (int f = 0; f < 4; f++) cs[f] = 0;
+    }
+}
+
 template <bool SEG>
-__global__ __launch_bounds__(256) void k_gather_sources_binned(DevPlan pl, DevSlabs sl, float4 *__restrict__ out,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned(DevPlan pl, DevSlabs sl, float4 *__restrict__ out,
                                                                float4 *__restrict__ box, float cpdf,
-                                                               double invcpd) {
+                                                               double invcpd, QueueClear qc) {
+    if (blockIdx.x == 0 && qc.counter) clear_queues(qc, threadIdx.x);
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x / kWave));
     if (w >= gather_waves(pl.nsrc_sets, pl.nsrc_blocks, pl.max_src_blocks) || plan_bad(pl)) return;
     gather_wave<SEG>(pl, sl, out, box, cpdf, invcpd, w, threadIdx.x & (kWave - 1));
@@ -478,9 +547,10 @@ __device__ __forceinline__ int group_sic_of(const int32_t *first, int n, int w) 
 // Every SIC's source gather of a launch group in one launch: a group of
 // small SICs (a clustered box's) fills the GPU where one SIC's pencils do not.
 template <bool SEG>
-__global__ __launch_bounds__(256) void k_gather_sources_binned_group(const GroupSic *__restrict__ g,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned_group(const GroupSic *__restrict__ g,
                                                                      const int32_t *__restrict__ first, int n,
-                                                                     float cpdf, double invcpd) {
+                                                                     float cpdf, double invcpd, QueueClear qc) {
+    if (blockIdx.x == 0 && qc.counter) clear_queues(qc, threadIdx.x);
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x / kWave));
     if (w >= cptr<int32_t>(first)[n]) return;
     const int i = group_sic_of(first, n, w);
@@ -673,37 +743,54 @@ __global__ __launch_bounds__(64) void k_plain(DevPlan pl, PairConst pc, FormRadi
     if (real) out[id] = make_float4(ax, ay, az, aw);
 }
 
+// The co-adds give a chunk (up to 64 particles of a sink cell) to LANES lanes:
+// a whole wave, or 16 lanes where cells hold few particles (launch_coadd_*).
+//
 // Addresses of the W partials of the sinks of cell (j_low + j, z): the cell is
-// at position c of pencil k = z - c (mod cpd).  Returns the cell's slab start
-// and count; base[c] is the padded slot of its first particle in pencil k.
-// and, if planes, split[c] the first of the cell's particles (its own numbering)
-// whose partial in pencil k is not spread over the source pencils' planes.
-__device__ __forceinline__ void partial_slots(const DevPlan &pl, int j, int z, int64_t *base, uint32_t *cstart,
-                                              int *cn, bool planes = false, int *split = nullptr) {
-    const int Nk = pl.Nk, W = pl.W, cpd = pl.cpd;
-    const nf_sink_plan &own = pl.sink_plan[j * Nk + z];  // pencil k = z starts with cell z
-    *cstart = own.cell[0].start;
-    *cn = own.cell[0].N;
-    for (int c = 0; c < W; c++) {
-        int k = z - c;
-        if (k < 0) k += cpd;
-        const int s = j * Nk + k;
-        const nf_sink_plan &pk = pl.sink_plan[s];
-        int off = 0;
-        for (int c2 = 0; c2 < c; c2++) off += pk.cell[c2].N;
-        base[c] = (int64_t)pl.sink_set_start[s] + off;
+// at position c of pencil k = z - c (mod cpd).  Lane c < W of the chunk's lanes
+// looks pencil k up, all of them at once (one lookup after the other took
+// 13 us of a 980-sink SIC's co-add).  base: the padded slot of the cell's first
+// particle in pencil k; with planes, split: the first of the cell's particles
+// (its own numbering) whose partial there is not spread over the source
+// pencils' planes.  Every lane gets the cell's slab start and its count (0 if
+// not `on`).  Every lane of the wave must call it.
+struct PartialSlots {
+    int base, split;  // lane c's
+    uint32_t cstart;
+    int cn;
+};
+template <int LANES>
+__device__ __forceinline__ PartialSlots partial_slots(const DevPlan &pl, bool on, int cell, int l, bool planes) {
+    const int z = cell % pl.Nk, c = min(l, pl.W - 1), k = z >= c ? z - c : z - c + pl.cpd;
+    const int s = cell - z + k;
+    PartialSlots p{0, 0, 0, 0};
+    int n = 0;
+    uint64_t nsrc = 0;
+    if (on) {
+        const nf_cell_plan own = pl.sink_plan[s].cell[0];  // pencil k starts with cell k = z - c
+        p.base = pl.sink_set_start[s];
+        p.cstart = own.start;
+        n = own.N;
         if (planes) {
-            uint64_t nsrc = 0;
-            for (int y = 0; y < W; y++) nsrc += (uint64_t)pl.src_set_count[pl.ilist[s * W + y]];
-            split[c] = y_split(nsrc, pl.y_cost) ? tile_sinks(pl.sink_set_count[s]) - off : 0;
+            p.split = pl.sink_set_count[s];
+#pragma unroll
+            for (int y = 0; y < NF_MAX_WIDTH; y++)
+                if (y < pl.W) nsrc += (uint64_t)pl.src_set_count[pl.ilist[s * pl.W + y]];
         }
     }
+    int off = 0;  // the pencil's cells before this one: cells z - c .. z - 1
+#pragma unroll
+    for (int i = 1; i < NF_MAX_WIDTH; i++) {
+        const int ni = __shfl(n, i, LANES);
+        off += c >= i ? ni : 0;
+    }
+    p.base += off;
+    p.split = planes && y_split(nsrc, pl.y_cost) ? tile_sinks(p.split) - off : 0;
+    p.cstart = __shfl(p.cstart, 0, LANES);
+    p.cn = __shfl(n, 0, LANES);
+    return p;
 }
 
-// FP32 co-add in the reference's order: the pencils of a skewer are applied
-// in increasing k, the first one setting the value and the rest adding.  For
-// cell z that is c = min(z, W-1) .. 0, then W-1 .. z+1.  One wave per chunk
-// of 64 particles of a sink cell.
 // RescaleAndCoAddAcceleration (kick.cpp:96-105) on one sink's float4, with
 // the FLOAT3p1 rules (float3p1.cpp:41-56): x, y, z = (a * inv_eps3 + far) *
 // rescale in float, each operation rounded on its own (no contraction), and
@@ -722,89 +809,116 @@ __device__ __forceinline__ float4 apply_kick(float4 a, const KickArgs &k, int64_
     return a;
 }
 
+// FP32 co-add in the reference's order: the pencils of a skewer are applied
+// in increasing k, the first one setting the value and the rest adding.  For
+// cell z that is c = min(z, W-1) .. 0, then W-1 .. z+1.
+template <int LANES>
 __global__ __launch_bounds__(256) void k_coadd_plain(DevPlan pl, const float4 *__restrict__ part,
                                                      float4 *__restrict__ acc, KickArgs kick) {
-    const int q = blockIdx.x * 4 + (int)(threadIdx.x / kWave);
-    if (q >= coadd_chunks(pl) || plan_bad(pl)) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int cell = pl.coadd_chunk[2 * q], first = pl.coadd_chunk[2 * q + 1];
-    const int j = cell / pl.Nk, z = cell % pl.Nk;
-    int64_t base[NF_MAX_WIDTH];
-    uint32_t cstart;
-    int cn;
-    partial_slots(pl, j, z, base, &cstart, &cn);
-    const int W = pl.W;
-    int order[NF_MAX_WIDTH], no = 0;
-    for (int c = (z < W - 1 ? z : W - 1); c >= 0; c--) order[no++] = c;
-    for (int c = W - 1; c > z; c--) order[no++] = c;
-    const int i = first + lane;
-    if (i >= cn) return;
-    float4 a = part[base[order[0]] + i];
-    for (int t = 1; t < W; t++) {
-        const float4 p = part[base[order[t]] + i];
-        a.x += p.x;
-        a.y += p.y;
-        a.z += p.z;
-        a.w += p.w;
+    const int q = (int)((blockIdx.x * 256 + threadIdx.x) / LANES), l = threadIdx.x % LANES;
+    const int nq = coadd_chunks(pl);
+    if ((int)(blockIdx.x * 256 + (threadIdx.x & ~(kWave - 1))) / LANES >= nq || plan_bad(pl)) return;
+    const bool on = q < nq;
+    const int cell = on ? pl.coadd_chunk[2 * q] : 0, first = on ? pl.coadd_chunk[2 * q + 1] : 0;
+    const PartialSlots ps = partial_slots<LANES>(pl, on, cell, l, false);
+    const int W = pl.W, m = min(cell % pl.Nk, W - 1);
+    int base[NF_MAX_WIDTH];  // in that order
+#pragma unroll
+    for (int t = 0; t < NF_MAX_WIDTH; t++) base[t] = __shfl(ps.base, t <= m ? m - t : max(W + m - t, 0), LANES);
+    for (int i = first + l, e = min(first + kWave, ps.cn); i < e; i += LANES) {
+        float4 a = part[base[0] + i];
+#pragma unroll
+        for (int t = 1; t < NF_MAX_WIDTH; t++) {
+            if (t >= W) break;
+            const float4 p = part[base[t] + i];
+            a.x += p.x;
+            a.y += p.y;
+            a.z += p.z;
+            a.w += p.w;
+        }
+        acc[ps.cstart + i] = apply_kick(a, kick, (int64_t)ps.cstart + i);
     }
-    acc[cstart + i] = apply_kick(a, kick, (int64_t)cstart + i);
 }
 
 // FP64 co-add: sum of the W double partials, scaled back to the reference's
-// units (out_scale applies to a, not to w).  One wave per 64-particle chunk.
+// units (out_scale applies to a, not to w).  q, l: the lane's chunk (on: it is
+// one) and its place among the chunk's lanes.  PLANES: the partials have planes
+// per source pencil; a launch that has them is small and waits for its loads,
+// so a sink's loads go out W partials at a time, a plane after the other (a
+// 980-sink SIC's co-add 13.5 -> 9.8 us; two planes at a time 8.7, but 29 instead
+// of 20 us for a group of eight 64^3 SICs, at 210 registers).
+template <int LANES, bool PLANES>
 __device__ __forceinline__ void coadd_chunk_f64(const DevPlan &pl, const double *__restrict__ part, double out_scale,
-                                                float4 *__restrict__ acc, const KickArgs &kick, int q, int lane) {
-    const int cell = pl.coadd_chunk[2 * q], first = pl.coadd_chunk[2 * q + 1];
-    const int j = cell / pl.Nk, z = cell % pl.Nk;
-    int64_t base[NF_MAX_WIDTH];
-    int split[NF_MAX_WIDTH];
-    uint32_t cstart;
-    int cn;
-    const int64_t plane = pl.y_plane;
-    partial_slots(pl, j, z, base, &cstart, &cn, plane != 0, split);
+                                                float4 *__restrict__ acc, const KickArgs &kick, int q, bool on,
+                                                int l) {
+    const int cell = on ? pl.coadd_chunk[2 * q] : 0, first = on ? pl.coadd_chunk[2 * q + 1] : 0;
+    const PartialSlots ps = partial_slots<LANES>(pl, on, cell, l, PLANES);
     const int W = pl.W;
-    const int i = first + lane;
-    if (i >= cn) return;
-    double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-    for (int c = 0; c < W; c++) {
-        const double *p = part + 4 * (base[c] + i);
-        double h0 = p[0], h1 = p[1], h2 = p[2], h3 = p[3];
-        if (plane != 0 && i < split[c])
-            for (int y = 1; y < W; y++) {
-                const double *q = p + y * plane;
-                h0 += q[0];
-                h1 += q[1];
-                h2 += q[2];
-                h3 += q[3];
-            }
-        a0 += h0;
-        a1 += h1;
-        a2 += h2;
-        a3 += h3;
+    int base[NF_MAX_WIDTH], split[NF_MAX_WIDTH];
+#pragma unroll
+    for (int c = 0; c < NF_MAX_WIDTH; c++) {
+        base[c] = __shfl(ps.base, c, LANES);
+        split[c] = PLANES ? __shfl(ps.split, c, LANES) : 0;
     }
-    const float4 a = make_float4((float)(a0 * out_scale), (float)(a1 * out_scale), (float)(a2 * out_scale), (float)a3);
-    acc[cstart + i] = apply_kick(a, kick, (int64_t)cstart + i);
+    for (int i = first + l, e = min(first + kWave, ps.cn); i < e; i += LANES) {
+        double h[NF_MAX_WIDTH][4];
+        auto partial = [&](int c, int y, double *out) {
+            const double *p =
+                part + 4 * ((int64_t)base[c < W ? c : 0] + i) + (y > 0 && y < W && i < split[c] ? y * pl.y_plane : 0);
+#pragma unroll
+            for (int t = 0; t < 4; t++) out[t] = p[t];
+        };
+#pragma unroll
+        for (int c = 0; c < NF_MAX_WIDTH; c++) partial(c, 0, h[c]);
+        if constexpr (PLANES)
+#pragma unroll
+            for (int y = 1; y < NF_MAX_WIDTH; y++) {
+                double g[NF_MAX_WIDTH][4];
+#pragma unroll
+                for (int c = 0; c < NF_MAX_WIDTH; c++) partial(c, y, g[c]);
+#pragma unroll
+                for (int c = 0; c < NF_MAX_WIDTH; c++)
+                    if (y < W && i < split[c])
+#pragma unroll
+                        for (int t = 0; t < 4; t++) h[c][t] += g[c][t];
+            }
+        double a[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < NF_MAX_WIDTH; c++) {
+            if (c >= W) break;
+#pragma unroll
+            for (int t = 0; t < 4; t++) a[t] += h[c][t];
+        }
+        const float4 r =
+            make_float4((float)(a[0] * out_scale), (float)(a[1] * out_scale), (float)(a[2] * out_scale), (float)a[3]);
+        acc[ps.cstart + i] = apply_kick(r, kick, (int64_t)ps.cstart + i);
+    }
 }
 
+template <int LANES, bool PLANES>
 __global__ __launch_bounds__(256) void k_coadd_f64(DevPlan pl, const double *__restrict__ part, double out_scale,
                                                    float4 *__restrict__ acc, KickArgs kick) {
-    const int q = blockIdx.x * 4 + (int)(threadIdx.x / kWave);
-    if (q >= coadd_chunks(pl) || plan_bad(pl)) return;
-    coadd_chunk_f64(pl, part, out_scale, acc, kick, q, threadIdx.x & (kWave - 1));
+    const int q = (int)((blockIdx.x * 256 + threadIdx.x) / LANES);
+    const int nq = coadd_chunks(pl);
+    if ((int)(blockIdx.x * 256 + (threadIdx.x & ~(kWave - 1))) / LANES >= nq || plan_bad(pl)) return;
+    coadd_chunk_f64<LANES, PLANES>(pl, part, out_scale, acc, kick, q, q < nq, threadIdx.x % LANES);
 }
 
 // Every SIC's FP64 co-add of a launch group in one launch.
+template <int LANES, bool PLANES>
 __global__ __launch_bounds__(256) void k_coadd_f64_group(const GroupSic *__restrict__ g,
                                                          const int32_t *__restrict__ first, int n) {
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x / kWave));
     if (w >= cptr<int32_t>(first)[n]) return;
     const int i = group_sic_of(first, n, w);
     const DevPlan pl = cptr<GroupSic>(g)[i].pl;
-    const int q = w - cptr<int32_t>(first)[i];
-    if (q >= coadd_chunks(pl) || plan_bad(pl)) return;
+    const int q0 = (w - cptr<int32_t>(first)[i]) * (kWave / LANES), nq = coadd_chunks(pl);
+    if (q0 >= nq || plan_bad(pl)) return;
+    const int lane = threadIdx.x & (kWave - 1), q = q0 + lane / LANES;
     const KickArgs kick = cptr<GroupSic>(g)[i].kick;
-    coadd_chunk_f64(pl, static_cast<const double *>(cptr<GroupSic>(g)[i].partial), cptr<GroupSic>(g)[i].out_scale,
-                    reinterpret_cast<float4 *>(cptr<GroupSic>(g)[i].acc4), kick, q, threadIdx.x & (kWave - 1));
+    coadd_chunk_f64<LANES, PLANES>(pl, static_cast<const double *>(cptr<GroupSic>(g)[i].partial),
+                                   cptr<GroupSic>(g)[i].out_scale, reinterpret_cast<float4 *>(cptr<GroupSic>(g)[i].acc4),
+                                   kick, q, q < nq, lane % LANES);
 }
 
 // ---------------------------------------------------------------------------
@@ -1229,16 +1343,18 @@ __device__ __forceinline__ void full_item(const BatchCtx &cx, const SicView &v, 
 // on L = ceil(r / 2) lanes, the wave holds G = 64 / L such groups, and group g
 // takes every G-th source of a block, from source g on.  One pass over the
 // sources whatever r is, all lanes busy but 64 - L G and one slot of an odd r.
-// The sources come through vector loads (one 16 B load per two pairs of a
-// lane, the same address on a group's lanes).  Each block's FP32 sums join
-// FP64 sums per lane, as a register tile's do, and a tree over the groups adds
-// those.
+// A block's 64 sources are loaded one to a lane, the next block's while this
+// one is summed, and handed to the groups through the wave's LDS (one 16 B read
+// per two pairs of a lane, the same address on a group's lanes).  Each block's
+// FP32 sums join FP64 sums per lane, as a register tile's do, and a tree over
+// the groups adds those.
 //
 // Against the sources on 16-lane groups with up to 8 sinks per pass, which this
 // replaces: the direct kernel of 24 sparse slabs (129^2 pencils of 25 sinks
 // each) 3.30 -> 1.27 ms, of eight 512^3 slabs 14.77 -> 14.08 ms (the tails
-// alone took 1.25 ms of that).  Two loads in flight (kAhead) instead of four
-// measured 0.5% faster but on the sparse slabs.
+// alone took 1.25 ms of that).  With every group loading its sources itself,
+// two loads ahead, a lone tail of 36 sinks and 500 sources took 35 us; through
+// LDS 23 us, and the sparse slabs 1.06 -> 0.97 ms.
 template <int SOFT, int MODE>
 __device__ __forceinline__ void tail_block(const float4 *bp, int cnt, int G, int full, int grp, const float *kx,
                                            const float *ky, const float *kz, const PairConst &pc, float *tx,
@@ -1255,7 +1371,7 @@ __device__ __forceinline__ void tail_block(const float4 *bp, int cnt, int G, int
         for (int u = 0; u < 2; u++)
             pair_sum(pair_g<SOFT, MODE>(r2[u], f[u], pc), dx[u], dy[u], dz[u], tx[u], ty[u], tz[u]);
     };
-    constexpr int kAhead = 2;  // loads in flight
+    constexpr int kAhead = 2;  // reads in flight
     int i = 0;
     for (; i + kAhead <= full; i += kAhead) {
         float4 sv[kAhead];
@@ -1264,23 +1380,18 @@ __device__ __forceinline__ void tail_block(const float4 *bp, int cnt, int G, int
 #pragma unroll
         for (int q = 0; q < kAhead; q++) pairs(sv[q]);
     }
-    if (i * G < cnt) {  // the last steps: a group past the block's sources takes a padding source
-        float4 sv[kAhead];
-#pragma unroll
-        for (int q = 0; q < kAhead; q++) sv[q] = bp[min((i + q) * G + grp, cnt - 1)];
-#pragma unroll
-        for (int q = 0; q < kAhead; q++) {
-            if ((i + q) * G >= cnt) break;
-            if ((i + q) * G + grp >= cnt) sv[q].x = kFar;
-            pairs(sv[q]);
-        }
+    for (; i * G < cnt; i++) {  // the last steps: a group past the block's sources takes a padding source
+        float4 sv = bp[min(i * G + grp, kWave - 1)];
+        if (i * G + grp >= cnt) sv.x = kFar;
+        pairs(sv);
     }
 }
 
+// block: the wave's 64 float4 in LDS.
 template <int SOFT, bool CENSUS>
-__device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, int lane,
-                                          Census &cen) {
-    const float4 *src = static_cast<const float4 *>(v.sources4);
+__device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, const WorkItem &w, float4 *block,
+                                          int lane, Census &cen) {
+    const NF_CONST float4 *src = cptr<float4>(v.sources4);
     NF_GLOBAL double *out = (NF_GLOBAL double *)v.partial;
     const int s = w.sinkset;
     const int base = cptr<int32_t>(v.sink_set_start)[s] + w.first;
@@ -1310,9 +1421,24 @@ __device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, 
     const SinkBox kbox = {wave_min(blx), wave_min(bly), wave_max(bhx), wave_max(bhy), blz, bhz, blz, bhz};
     double h[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
     const int W = v.W, full64 = kWave / G;
+    // The next block's sources, one to a lane: from block `at` on (the blocks
+    // of a pencil follow each other; ny, nleft: its pencil and blocks to come).
+    int ny = -1, nleft = 0, at = 0;
+    float4 ahead = make_float4(kFar, 0.f, 0.f, 0.f);
+    auto load_next = [&] {
+        while (nleft == 0 && ++ny < W) {
+            nleft = (rows.count_of(ny) + kWave - 1) / kWave;
+            at = rows.start_of(ny);
+        }
+        if (ny >= W) return;
+        ahead = src[at + lane];
+        at += kWave;
+        nleft--;
+    };
+    load_next();
     int modes = 0, p = 0;
     for (int y = 0; y < W; y++) {
-        const int st = rows.start_of(y), n = rows.count_of(y);
+        const int n = rows.count_of(y);
         const double yo = (double)(y - v.R) * cx.invcpd;
         float kyy[2];
 #pragma unroll
@@ -1326,7 +1452,13 @@ __device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, 
                 census_add(cen, mode, (uint64_t)r * (uint64_t)cnt);
                 cen.tail += (uint64_t)r * (uint64_t)cnt;
             }
-            const float4 *bp = src + st + b * kWave;
+            // (LDS is in order within the wave: the block's reads follow its
+            // write, and the next block's write follows them.)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            block[lane] = ahead;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            load_next();
+            const float4 *bp = block;
             const int full = cnt == kWave ? full64 : cnt / G;
             float tx[2] = {0.f, 0.f}, ty[2] = {0.f, 0.f}, tz[2] = {0.f, 0.f}, tw[2] = {0.f, 0.f};
             if (mode == kNoDensity)
@@ -1397,8 +1529,6 @@ namespace {
 // out item by item, so they end within about an item of each other.  (Dealing
 // it to one queue per XCD in chunks of 8 to 128 consecutive items, which share
 // source pencils, measured 11% slower.)
-constexpr int kCensusOffset = kCensusBytes / 4;  // int32 units
-constexpr int kQueueOffset = kQueueBytes / 4, kQueueStride = kQueueLine / 4;
 template <int SOFT, int S, int WPE, bool CENSUS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_batched(
     BatchCtx cx, const SicView *__restrict__ views, const WorkItem *__restrict__ items, int32_t nitems,
@@ -1430,26 +1560,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
         } else if (kind >= 2) {  // one-wave tiles, whole or against one source pencil
             const int y = w.nsink >> 8;
             full_item<SOFT, 1, CENSUS>(cx, v, w, w.nsink & 255, y, kind == 2 ? v.W : y + 1, hsum, lane, cen);
-        } else tail_item<SOFT, CENSUS>(cx, v, w, lane, cen);
+        } else tail_item<SOFT, CENSUS>(cx, v, w, reinterpret_cast<float4 *>(hsum - lane), lane, cen);
         int j = 0;
         if (lane == 0) j = atomicAdd(counter + kQueueOffset + q * kQueueStride, 1);
         it = nwaves + __builtin_amdgcn_readfirstlane(j) * nq + q;
     }
 }
 
-// The batched launch's prologue (a fill kernel, so that it can sit in a
-// captured graph): clears the queues and, for a census build, the census; for a device-planned list, copies its length into counter[1], or
-// 0 when the group holds a cell outside its slab.
-__global__ void k_zero_counter(int32_t *c, const int32_t *dnitems, const int32_t *dbad, int census) {
-    const int t = threadIdx.x;
-    if (t < kQueues) c[kQueueOffset + t * kQueueStride] = 0;
-    if (t != 0) return;
-    if (dnitems) c[1] = (dbad && *dbad != 0) ? 0 : *dnitems;
-    if (census) {
-        unsigned long long *cs = reinterpret_cast<unsigned long long *>(c + kCensusOffset);
-        for (int f = 0; f < 4; f++) cs[f] = 0;
-    }
-}
+// The batched launch's prologue where no gather before it cleared the queues
+// (a kernel, so that it can sit in a captured graph).
+__global__ void k_zero_counter(QueueClear qc) { clear_queues(qc, threadIdx.x); }
 
 // Pair-math probe: the register-tile loop of k_batched alone (16-source batch
 // sums, 64-source FP32 tile sums accumulated in FP64), one pair form for
@@ -1555,7 +1675,7 @@ int device_cu_count() {
 }
 
 int launch_gather(const DevPlan &pl, const DevSlabs &sl, bool batched_stream, void *sinks4, void *sources4,
-                  void *stream) {
+                  const QueueClear &qc, void *stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     const float cellsize = (float)(1.0 / (double)pl.cpd);
     const double invcpd = 1.0 / (double)pl.cpd;
@@ -1574,10 +1694,10 @@ int launch_gather(const DevPlan &pl, const DevSlabs &sl, bool batched_stream, vo
             const dim3 bgrid((unsigned)((gather_waves(pl.nsrc_sets, pl.nsrc_blocks, pl.max_src_blocks) + 3) / 4));
             if (gather_segmented(pl.max_src_blocks))
                 hipLaunchKernelGGL(k_gather_sources_binned<true>, bgrid, dim3(256), 0, st, pl, sl,
-                                   static_cast<float4 *>(sources4), box, (float)pl.cpd, invcpd);
+                                   static_cast<float4 *>(sources4), box, (float)pl.cpd, invcpd, qc);
             else
                 hipLaunchKernelGGL(k_gather_sources_binned<false>, bgrid, dim3(256), 0, st, pl, sl,
-                                   static_cast<float4 *>(sources4), box, (float)pl.cpd, invcpd);
+                                   static_cast<float4 *>(sources4), box, (float)pl.cpd, invcpd, qc);
         }
         else
             hipLaunchKernelGGL(k_gather_sources, grid, dim3(256), 0, st, pl, sl, static_cast<float4 *>(sources4),
@@ -1587,23 +1707,26 @@ int launch_gather(const DevPlan &pl, const DevSlabs &sl, bool batched_stream, vo
 }
 
 int launch_gather_group(const GroupSic *g, const int32_t *first, int n, int total, int cpd, bool segmented,
-                        void *stream) {
+                        const QueueClear &qc, void *stream) {
     if (total <= 0) return 0;
     const dim3 grid((unsigned)((total + 3) / 4));
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (segmented)
         hipLaunchKernelGGL(k_gather_sources_binned_group<true>, grid, dim3(256), 0, st, g, first, n, (float)cpd,
-                           1.0 / (double)cpd);
+                           1.0 / (double)cpd, qc);
     else
         hipLaunchKernelGGL(k_gather_sources_binned_group<false>, grid, dim3(256), 0, st, g, first, n, (float)cpd,
-                           1.0 / (double)cpd);
+                           1.0 / (double)cpd, qc);
     return (int)hipGetLastError();
 }
 
-int launch_coadd_group(const GroupSic *g, const int32_t *first, int n, int total, void *stream) {
+int launch_coadd_group(const GroupSic *g, const int32_t *first, int n, int total, int lanes, bool planes,
+                       void *stream) {
     if (total <= 0) return 0;
-    hipLaunchKernelGGL(k_coadd_f64_group, dim3((unsigned)((total + 3) / 4)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), g, first, n);
+    const auto kern = lanes == 16 ? (planes ? k_coadd_f64_group<16, true> : k_coadd_f64_group<16, false>)
+                                  : (planes ? k_coadd_f64_group<64, true> : k_coadd_f64_group<64, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(stream), g,
+                       first, n);
     return (int)hipGetLastError();
 }
 
@@ -1622,27 +1745,34 @@ int launch_plain(const DevPlan &pl, int softening, const PairConst &pc, const vo
     }
 }
 
-int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, const KickArgs &kick, void *stream) {
+int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, const KickArgs &kick, int lanes,
+                       void *stream) {
     if (pl.n_coadd_chunks == 0) return 0;
+    const dim3 grid((unsigned)((group_coadd_waves(pl, lanes) + 3) / 4));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_coadd_plain, dim3((pl.n_coadd_chunks + 3) / 4), dim3(256), 0, st, pl,
-                       static_cast<const float4 *>(partial4), reinterpret_cast<float4 *>(acc4), kick);
+    const float4 *part = static_cast<const float4 *>(partial4);
+    float4 *acc = reinterpret_cast<float4 *>(acc4);
+    if (lanes == 16) hipLaunchKernelGGL(k_coadd_plain<16>, grid, dim3(256), 0, st, pl, part, acc, kick);
+    else hipLaunchKernelGGL(k_coadd_plain<64>, grid, dim3(256), 0, st, pl, part, acc, kick);
     return (int)hipGetLastError();
 }
 
 int launch_coadd_f64(const DevPlan &pl, const void *partial_d4, double out_scale, float *acc4,
-                     const KickArgs &kick, void *stream) {
+                     const KickArgs &kick, int lanes, void *stream) {
     if (pl.n_coadd_chunks == 0) return 0;
+    const dim3 grid((unsigned)((group_coadd_waves(pl, lanes) + 3) / 4));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_coadd_f64, dim3((pl.n_coadd_chunks + 3) / 4), dim3(256), 0, st, pl,
-                       static_cast<const double *>(partial_d4), out_scale, reinterpret_cast<float4 *>(acc4), kick);
+    const bool planes = pl.y_plane != 0;
+    const auto kern = lanes == 16 ? (planes ? k_coadd_f64<16, true> : k_coadd_f64<16, false>)
+                                  : (planes ? k_coadd_f64<64, true> : k_coadd_f64<64, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, pl, static_cast<const double *>(partial_d4), out_scale,
+                       reinterpret_cast<float4 *>(acc4), kick);
     return (int)hipGetLastError();
 }
 
 template <int SOFT, int S, bool CENSUS>
 static int launch_batched_k(const BatchCtx &cx, const TileShape &ts, const SicView *views, const WorkItem *items,
-                            int32_t nitems, int32_t *counter, hipStream_t st, const int32_t *dnitems,
-                            const int32_t *dbad) {
+                            int32_t nitems, const QueueClear &qc, bool cleared, hipStream_t st) {
     constexpr auto kern = k_batched<SOFT, S, batched_waves_per_eu(SOFT, S), CENSUS>;
     // Workgroups of 1, 2 or 4 waves; each wave pops its own items, so the
     // size only changes how the dispatcher places the persistent grid.
@@ -1659,27 +1789,26 @@ static int launch_batched_k(const BatchCtx &cx, const TileShape &ts, const SicVi
     const int need = (nitems + wpw - 1) / wpw;
     if (grid > need) grid = std::max(1, need);
     static_assert(kCensusBytes + 32 <= kQueueBytes && kQueues <= kWave, "census before the queues, one lane per queue");
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(kWave), 0, st, counter, dnitems, dbad, CENSUS ? 1 : 0);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, st, cx, views, items, dnitems ? -nitems : nitems, counter);
+    if (!cleared) hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(kWave), 0, st, qc);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, st, cx, views, items, qc.dnitems ? -nitems : nitems,
+                       qc.counter);
     return (int)hipGetLastError();
 }
 
 template <int SOFT, int S>
 static int launch_batched_s(const BatchCtx &cx, const TileShape &ts, const SicView *views, const WorkItem *items,
-                            int32_t nitems, int32_t *counter, hipStream_t st, const int32_t *dnitems,
-                            const int32_t *dbad, bool census) {
-    if (census) return launch_batched_k<SOFT, S, true>(cx, ts, views, items, nitems, counter, st, dnitems, dbad);
-    return launch_batched_k<SOFT, S, false>(cx, ts, views, items, nitems, counter, st, dnitems, dbad);
+                            int32_t nitems, const QueueClear &qc, bool cleared, hipStream_t st) {
+    if (qc.census) return launch_batched_k<SOFT, S, true>(cx, ts, views, items, nitems, qc, cleared, st);
+    return launch_batched_k<SOFT, S, false>(cx, ts, views, items, nitems, qc, cleared, st);
 }
 
 template <int SOFT>
 static int launch_batched_soft(const BatchCtx &cx, const TileShape &ts, const SicView *views, const WorkItem *items,
-                               int32_t nitems, int32_t *counter, hipStream_t st, const int32_t *dnitems,
-                               const int32_t *dbad, bool census) {
+                               int32_t nitems, const QueueClear &qc, bool cleared, hipStream_t st) {
     switch (ts.sinks_per_lane) {
-        case 1: return launch_batched_s<SOFT, 1>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
-        case 2: return launch_batched_s<SOFT, 2>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
-        case 4: return launch_batched_s<SOFT, 4>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
+        case 1: return launch_batched_s<SOFT, 1>(cx, ts, views, items, nitems, qc, cleared, st);
+        case 2: return launch_batched_s<SOFT, 2>(cx, ts, views, items, nitems, qc, cleared, st);
+        case 4: return launch_batched_s<SOFT, 4>(cx, ts, views, items, nitems, qc, cleared, st);
         default: return (int)hipErrorInvalidValue;
     }
 }
@@ -1701,8 +1830,7 @@ int run_pair_probe(const PairConst &pc, int sinks_per_lane, int mode, int waves_
 }
 
 int launch_batched(const SicView *views, int cpd, int softening, const PairConst &pc, const TileShape &ts,
-                   const WorkItem *items, int32_t nitems, int32_t *counter, void *stream, const int32_t *dnitems,
-                   const int32_t *dbad, bool census) {
+                   const WorkItem *items, int32_t nitems, const QueueClear &qc, bool cleared, void *stream) {
     if (nitems == 0) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     BatchCtx cx;
@@ -1710,13 +1838,13 @@ int launch_batched(const SicView *views, int cpd, int softening, const PairConst
     cx.invcpd = 1.0 / (double)cpd;
     cx.fr = form_radii(softening, pc, pc.b2x);  // (density is nonzero only for r^2 + r2add < b2x)
     switch (softening) {
-        case NF_SOFT_PLUMMER: return launch_batched_soft<NF_SOFT_PLUMMER>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
+        case NF_SOFT_PLUMMER: return launch_batched_soft<NF_SOFT_PLUMMER>(cx, ts, views, items, nitems, qc, cleared, st);
         case NF_SOFT_SINGLE_SPLINE:
-            return launch_batched_soft<NF_SOFT_SINGLE_SPLINE>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
+            return launch_batched_soft<NF_SOFT_SINGLE_SPLINE>(cx, ts, views, items, nitems, qc, cleared, st);
         case NF_SOFT_CUBIC_SPLINE:
-            return launch_batched_soft<NF_SOFT_CUBIC_SPLINE>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
+            return launch_batched_soft<NF_SOFT_CUBIC_SPLINE>(cx, ts, views, items, nitems, qc, cleared, st);
         case NF_SOFT_CUBIC_PLUMMER:
-            return launch_batched_soft<NF_SOFT_CUBIC_PLUMMER>(cx, ts, views, items, nitems, counter, st, dnitems, dbad, census);
+            return launch_batched_soft<NF_SOFT_CUBIC_PLUMMER>(cx, ts, views, items, nitems, qc, cleared, st);
         default: return (int)hipErrorInvalidValue;
     }
 }

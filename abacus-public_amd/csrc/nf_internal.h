@@ -171,32 +171,40 @@ struct TileShape {
 // batched_stream the sources take FP64 cell offsets and each cell's particles
 // are ordered by x-bin (tighter block boxes); otherwise the reference's
 // order and FLOAT offsets.
+// The queues that a batched launch after a batched-path gather needs cleared
+// (counter null: none); the gather clears them if it has any source pencil.
+struct QueueClear {
+    int32_t *counter;         // the slot: see launch_batched
+    const int32_t *dnitems, *dbad;
+    int32_t census;
+};
 int launch_gather(const DevPlan &pl, const DevSlabs &sl, bool batched_stream, void *sinks4,
-                  void *sources4, void *stream);
+                  void *sources4, const QueueClear &qc, void *stream);
 int launch_plain(const DevPlan &pl, int softening, const PairConst &pc, const void *sinks4,
                  const void *sources4, void *partial4, void *stream);
-int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, const KickArgs &kick, void *stream);
+int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, const KickArgs &kick, int lanes,
+                       void *stream);
 // One persistent launch over the work items of a group of SICs.  With
-// dnitems (device memory) non-null the list holds *dnitems items and nitems
-// is only its bound; with dbad non-null and *dbad != 0 the kernel does
-// nothing.  counter names a slot of kCounterBytes: the device list's length
-// (int32 1), with census four uint64 at kCensusBytes receiving the pair
-// interactions computed in each pair form (unsoftened, with density, softened)
-// and, in the fourth, those of short tails (also counted by form), by a
-// diagnostic build of the kernel; and kQueues queue counters from kQueueBytes,
-// kQueueLine bytes apart.
+// qc.dnitems (device memory) non-null the list holds *qc.dnitems items and
+// nitems is only its bound; with qc.dbad non-null and *qc.dbad != 0 the kernel
+// does nothing.  qc.counter names a slot of kCounterBytes: the device list's
+// length (int32 1), with qc.census four uint64 at kCensusBytes receiving the
+// pair interactions computed in each pair form (unsoftened, with density,
+// softened) and, in the fourth, those of short tails (also counted by form), by
+// a diagnostic build of the kernel; and kQueues queue counters from
+// kQueueBytes, kQueueLine bytes apart.  cleared: a gather on the same stream has
+// cleared the slot.
 constexpr int kCensusBytes = 64;
 constexpr int kQueues = 16, kQueueBytes = 256, kQueueLine = 256;
 constexpr int kCounterBytes = kQueueBytes + kQueues * kQueueLine;
 int launch_batched(const SicView *views, int cpd, int softening, const PairConst &pc, const TileShape &ts,
-                   const WorkItem *items, int32_t nitems, int32_t *counter, void *stream,
-                   const int32_t *dnitems = nullptr, const int32_t *dbad = nullptr, bool census = false);
+                   const WorkItem *items, int32_t nitems, const QueueClear &qc, bool cleared, void *stream);
 // Bounding boxes follow a padded source stream of nsrc_blocks blocks.
 inline void *box_after(void *sources4, int32_t nsrc_blocks) {
     return static_cast<char *>(sources4) + (size_t)nsrc_blocks * NF_BLOCK_SIZE * 16;
 }
 int launch_coadd_f64(const DevPlan &pl, const void *partial_d4, double out_scale, float *acc4,
-                     const KickArgs &kick, void *stream);
+                     const KickArgs &kick, int lanes, void *stream);
 // One SIC of a launch group, for the group-wide batched-path gather and
 // co-add launches (device memory, beside the group's view table).
 struct GroupSic {
@@ -209,8 +217,8 @@ struct GroupSic {
     double out_scale;
 };
 // Waves of each SIC in the group-wide launches: the gather takes one per
-// source pencil, the co-add one per 64-particle chunk (its bound, for a
-// device-planned SIC).
+// source pencil, the co-add one per 64-particle chunk or per four of them (of
+// its bound, for a device-planned SIC).
 // Waves of a SIC's binned source gather: one per source pencil and, when a
 // pencil may have more than kGatherSegBlocks blocks, one per
 // kGatherSegBlocks blocks of the stream (the pencil waves then fill their
@@ -223,14 +231,22 @@ constexpr int32_t gather_waves(int32_t nsrc_sets, int32_t nsrc_blocks, int32_t m
 inline int32_t group_gather_waves(const DevPlan &pl) {
     return gather_waves(pl.nsrc_sets, pl.nsrc_blocks, pl.max_src_blocks);
 }
-inline int32_t group_coadd_waves(const DevPlan &pl) { return pl.n_coadd_chunks; }
+// The co-adds' lanes per chunk (up to 64 particles of a sink cell): 16 below 32
+// particles per cell, where a wave per chunk leaves most lanes idle (a group of
+// sparse SICs, 5 per cell: 94 -> 30 us on average), else 64.
+constexpr int coadd_lanes(uint64_t sinks, uint64_t cells) { return sinks < 32 * cells ? 16 : 64; }
+inline int32_t group_coadd_waves(const DevPlan &pl, int lanes) {
+    return (int32_t)(((int64_t)pl.n_coadd_chunks * lanes + 63) / 64);
+}
 // The batched-path source gathers of n SICs as one launch, then (a second
 // call) their FP64 co-adds as one launch.  first[i] is the first wave of SIC
 // i and first[n] the total (device memory, like g).
 // segmented: some SIC of the group has gather_segmented(max_src_blocks).
 int launch_gather_group(const GroupSic *g, const int32_t *first, int n, int total, int cpd, bool segmented,
-                        void *stream);
-int launch_coadd_group(const GroupSic *g, const int32_t *first, int n, int total, void *stream);
+                        const QueueClear &qc, void *stream);
+// planes: some SIC's partials have planes.
+int launch_coadd_group(const GroupSic *g, const int32_t *first, int n, int total, int lanes, bool planes,
+                       void *stream);
 // The single-spline pair-math probe (the batched tile loop alone, one pair
 // form: 0 unsoftened without density, 1 with density, 2 the full spline) at
 // a tile of S sinks per lane and an occupancy of waves_per_simd (4, 6 or 8):

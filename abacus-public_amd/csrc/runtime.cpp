@@ -1360,6 +1360,14 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     GroupSic *gsic = reinterpret_cast<GroupSic *>(hp + o_gsic);
     int32_t *gfirst = reinterpret_cast<int32_t *>(hp + o_gfirst), *cfirst = gfirst + (n + 1);
     gfirst[0] = cfirst[0] = 0;
+    uint64_t sinks = 0, cells = 0;
+    for (Task *t : g) {
+        uint64_t r0, r1;
+        task_rows(*t, &r0, &r1);
+        sinks += r1 > r0 ? r1 - r0 : 0;
+        cells += (uint64_t)t->sic.NSinkSets;
+    }
+    const int clanes = coadd_lanes(sinks, cells);
     for (int i = 0; i < n; i++) {
         GroupSic &G = gsic[i];
         std::memset(&G, 0, sizeof(G));
@@ -1371,7 +1379,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         G.acc4 = accd[i];
         G.out_scale = pc.out_scale;
         gfirst[i + 1] = gfirst[i] + group_gather_waves(plans[i]);
-        cfirst[i + 1] = cfirst[i] + group_coadd_waves(plans[i]);
+        cfirst[i + 1] = cfirst[i] + group_coadd_waves(plans[i], clanes);
     }
     for (size_t k = 0; k < itemsets.size(); k++)
         if (!itemsets[k]->empty())
@@ -1482,34 +1490,35 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     int e = 0;
     const GroupSic *gsic_d = reinterpret_cast<const GroupSic *>(pd + o_gsic);
     const int32_t *gfirst_d = reinterpret_cast<const int32_t *>(pd + o_gfirst), *cfirst_d = gfirst_d + (n + 1);
+    // The batched launch's queues, cleared by the gather.  A device-planned
+    // group's list lengths and bad cells are in its shared planning area.
+    const int32_t *gshared =
+        dplan ? reinterpret_cast<const int32_t *>(static_cast<char *>(w.gscratch.p) + gs.o_shared) : nullptr;
+    auto queues = [&](const TileShape &shape) {
+        const int ti = shape.sinks_per_lane == 1 ? 0 : shape.sinks_per_lane == 2 ? 1 : 2;
+        return QueueClear{reinterpret_cast<int32_t *>(pd + o_counter), gshared ? gshared + kPlanGroupItems + ti : nullptr,
+                          gshared ? gshared + kPlanGroupBad : nullptr, rt.params.census ? 1 : 0};
+    };
     if (path == NF_PATH_BATCHED) {
         bool seg = false;
         for (int i = 0; i < n; i++) seg = seg || gather_segmented(plans[i].max_src_blocks);
-        e = launch_gather_group(gsic_d, gfirst_d, n, gfirst[n], s0.cpd, seg, stream);
+        e = launch_gather_group(gsic_d, gfirst_d, n, gfirst[n], s0.cpd, seg, queues(ts), stream);
     }
     else
         for (int i = 0; i < n && !e; i++)
-            e = launch_gather(plans[i], slabs[i], false, wb + WL[i].o_sinks, wb + WL[i].o_src, stream);
+            e = launch_gather(plans[i], slabs[i], false, wb + WL[i].o_sinks, wb + WL[i].o_src, QueueClear{}, stream);
     if (e) return fail(NF_ERR_HIP, std::string("gather launch: ") + hipGetErrorString((hipError_t)e));
     if (!use_graph) NF_HIP(hipEventRecord(w.ev[2], stream));
     std::vector<hipEvent_t> tev;
     unsigned long long *census = nullptr;  // batched path: interactions per pair form (device)
     if (path == NF_PATH_BATCHED) {
-        int32_t *counter = reinterpret_cast<int32_t *>(pd + o_counter);
         if (rt.params.census)  // in the counter's slot
             census = reinterpret_cast<unsigned long long *>(pd + o_counter + kCensusBytes);
-        // A device-planned group's list lengths and bad cells are in its
-        // shared planning area.
-        const int32_t *gshared =
-            dplan ? reinterpret_cast<const int32_t *>(static_cast<char *>(w.gscratch.p) + gs.o_shared) : nullptr;
         auto launch = [&](const TileShape &shape) {
-            const int k = items_of(shape.sinks_per_lane);
-            const int ti = shape.sinks_per_lane == 1 ? 0 : shape.sinks_per_lane == 2 ? 1 : 2;
             return launch_batched(reinterpret_cast<const SicView *>(pd + o_views), s0.cpd, s0.softening, pc, shape,
-                                  reinterpret_cast<const WorkItem *>(pd + o_itemset[k]),
-                                  (int32_t)nitems[k], counter, stream,
-                                  gshared ? gshared + kPlanGroupItems + ti : nullptr,
-                                  gshared ? gshared + kPlanGroupBad : nullptr, census != nullptr);
+                                  reinterpret_cast<const WorkItem *>(pd + o_itemset[items_of(shape.sinks_per_lane)]),
+                                  (int32_t)nitems[items_of(shape.sinks_per_lane)], queues(shape),
+                                  !trial && gfirst[n] > 0, stream);
         };
         if (trial) {
             // Time each candidate; the chosen shape runs last (every candidate
@@ -1536,10 +1545,10 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     if (e) return fail(NF_ERR_HIP, std::string("direct kernel launch: ") + hipGetErrorString((hipError_t)e));
     if (!use_graph) NF_HIP(hipEventRecord(w.ev[3], stream));
     if (path == NF_PATH_BATCHED)
-        e = launch_coadd_group(gsic_d, cfirst_d, n, cfirst[n], stream);
+        e = launch_coadd_group(gsic_d, cfirst_d, n, cfirst[n], clanes, y_cost != UINT64_MAX, stream);
     else
         for (int i = 0; i < n && !e; i++)
-            e = launch_coadd_plain(plans[i], wb + WL[i].o_part, accd[i], kicks[i], stream);
+            e = launch_coadd_plain(plans[i], wb + WL[i].o_part, accd[i], kicks[i], clanes, stream);
     if (e) return fail(NF_ERR_HIP, std::string("co-add launch: ") + hipGetErrorString((hipError_t)e));
     if (use_graph) {
         hipGraph_t graph = nullptr;
@@ -2477,16 +2486,21 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     v.R = s.nfradius;
 
     // Upload, gather, one persistent launch, co-add, on the caller's stream;
-    // the queue counter is cleared by a kernel inside launch_batched.  The
+    // the gather clears the queues.  The
     // host image stays untouched until the stream has drained.
     hipStream_t st = static_cast<hipStream_t>(stream);
     NF_HIP(hipMemcpyAsync(d, h, L.image, hipMemcpyHostToDevice, st));
-    int e = launch_gather(pl, sl, true, nullptr, src, st);
+    const QueueClear qc{reinterpret_cast<int32_t *>(d + L.o_counter), nullptr, nullptr, 0};
+    int e = launch_gather(pl, sl, true, nullptr, src, qc, st);
     if (!e)
         e = launch_batched(reinterpret_cast<const SicView *>(d), s.cpd, s.softening, pc, TileShape{S, 64, 4, 0},
-                           reinterpret_cast<const WorkItem *>(d + L.o_items), (int32_t)nitems,
-                           reinterpret_cast<int32_t *>(d + L.o_counter), st);
-    if (!e) e = launch_coadd_f64(pl, d + L.work.o_part, pc.out_scale, s.SinkAccSlab, ka, st);
+                           reinterpret_cast<const WorkItem *>(d + L.o_items), (int32_t)nitems, qc,
+                           s.NSourceBlocks > 0, st);
+    uint64_t r0, r1;
+    sink_rows(s, &r0, &r1);
+    if (!e)
+        e = launch_coadd_f64(pl, d + L.work.o_part, pc.out_scale, s.SinkAccSlab, ka,
+                             coadd_lanes(r1 > r0 ? r1 - r0 : 0, (uint64_t)s.NSinkSets), st);
     const hipError_t se = hipStreamSynchronize(st);
     if (e) return fail(NF_ERR_HIP, std::string("nf_execute_sic_noalloc launch: ") + hipGetErrorString((hipError_t)e));
     if (se != hipSuccess) return fail(NF_ERR_HIP, std::string("nf_execute_sic_noalloc: ") + hipGetErrorString(se));
