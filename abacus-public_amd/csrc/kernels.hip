@@ -1001,10 +1001,21 @@ __device__ __forceinline__ void pair_box(float sx, float sy, float sz, float kx,
     pair_sum(pair_g<SOFT, MODE>(r2, f, pc), dx, dy, dz, ax, ay, az);
 }
 
+// Four sources in scalar registers, by one load.
+struct Sources4 {
+    float4 s[4];
+    __device__ __forceinline__ void load(const NF_CONST float4 *p) {
+        typedef float Float16 __attribute__((ext_vector_type(16)));
+        const Float16 v = *(const NF_CONST Float16 *)p;
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], 0.f);
+    }
+};
+
 // The pairs of P sources (at sp) with the S sinks of a lane, sink slots below
 // S/2 in form MLO and the others in MHI.
-template <int SOFT, int MLO, int MHI, int S, int P>
-__device__ __forceinline__ void pair_group(const NF_CONST float4 *sp, const float *kx, const float *ky,
+template <int SOFT, int MLO, int MHI, int S, int P, typename SrcP>
+__device__ __forceinline__ void pair_group(SrcP sp, const float *kx, const float *ky,
                                            const float *kz, const PairConst &pc, float *bx, float *by, float *bz,
                                            float *tw) {
     constexpr int N = P * S;
@@ -1155,6 +1166,19 @@ __device__ __forceinline__ void census_add(Census &c, int mode, uint64_t n) {
 // which code runs, not the result.  The last batch stops at the first multiple
 // of 4 past the cnt % kSrcBatch real sources: the padding sources give exact
 // zeros, so how many of them are taken changes no sum.
+//
+// The sources of full batches come four to a scalar load, the next four asked
+// for before these are summed: left to itself the compiler loads two sources
+// some 10 to 25 instructions before it waits for them, and the scalar cache
+// misses on most (a pencil is read once per item).  One batch stands in the
+// code, not the four of a block: the nine form pairs at S = 2 are 60 KB of the
+// 64 KB that two CUs' instruction cache holds, unrolled 87 KB.  Direct kernel
+// of eight 512^3 slabs at S = 1 / 2 / 4: 15.24 / 14.08 / 15.30 -> 14.13 / 13.66
+// / 14.64 ms; of radius-1 slabs with 512 particles a cell 8.97 / 8.91 / 11.19
+// -> 8.44 / 8.45 / 9.17 ms.  (The 512^3 slabs at S = 2 otherwise: unrolled
+// 13.77; eight sources a load, which spills scalar registers, 14.71; half a
+// batch in the code 13.83; the remainder in the same loop 14.39; sources
+// through LDS 14.11.)
 constexpr int kSrcBatch = 16;
 template <int SOFT, int MLO, int MHI, int S>
 __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, const float *kx, const float *ky,
@@ -1162,13 +1186,22 @@ __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, co
                                           float *tw) {
     constexpr int P = S == 1 ? 2 : 1;  // sources per pair_group
     const int fullb = cnt & ~(kSrcBatch - 1);
+    Sources4 sb[2];
+    if (fullb > 0) sb[0].load(sp);
+#pragma unroll 1
     for (int i = 0; i < fullb; i += kSrcBatch) {
         float bx[S], by[S], bz[S];
 #pragma unroll
         for (int u = 0; u < S; u++) bx[u] = by[u] = bz[u] = 0.f;
 #pragma unroll
-        for (int q = 0; q < kSrcBatch; q += P)
-            pair_group<SOFT, MLO, MHI, S, P>(sp + i + q, kx, ky, kz, pc, bx, by, bz, tw);
+        for (int h = 0; h < kSrcBatch / 4; h++) {
+            // (after a whole block's last batch the first sources again: in bounds, not used)
+            sb[(h + 1) & 1].load(sp + (h < kSrcBatch / 4 - 1 ? i + 4 * h + 4 : (i + kSrcBatch) % kWave));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 4; q += P)
+                pair_group<SOFT, MLO, MHI, S, P>(sb[h & 1].s + q, kx, ky, kz, pc, bx, by, bz, tw);
+        }
 #pragma unroll
         for (int u = 0; u < S; u++) {
             tx[u] += bx[u];
@@ -1181,6 +1214,7 @@ __device__ __forceinline__ void full_tile(const NF_CONST float4 *sp, int cnt, co
 #pragma unroll
         for (int u = 0; u < S; u++) bx[u] = by[u] = bz[u] = 0.f;
         // (by 4, the last of them padding: one wait for scalar loads per 4 sources)
+#pragma unroll 1
         for (int q = fullb; q < cnt; q += 4)
 #pragma unroll
             for (int k = 0; k < 4; k += P)
