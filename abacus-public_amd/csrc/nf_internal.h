@@ -158,7 +158,7 @@ int derive_pair_const(int softening, float eps, float b2, PairConst *pc);
 // a sink's sum does not depend on which lane, wave or workgroup computes it.
 struct TileShape {
     int sinks_per_lane;   // S: 1, 2 or 4
-    int tile;             // TwoSum tile depth in sources (sinks on lanes)
+    int tile;             // source tile depth
     int rem_sinks;        // uniform sinks per pass in the remainder path
     int waves_per_cu;     // persistent grid size (0: from occupancy)
     int waves_per_wg;     // workgroup size in waves: 1, 2 or 4 (0: 4)
@@ -197,6 +197,10 @@ int launch_coadd_plain(const DevPlan &pl, const void *partial4, float *acc4, con
 constexpr int kCensusBytes = 64;
 constexpr int kQueues = 16, kQueueBytes = 256, kQueueLine = 256;
 constexpr int kCounterBytes = kQueueBytes + kQueues * kQueueLine;
+// The queues are not counted against a scratch limit (a launch has one
+// counter block, beside the limit's bytes): a SIC that fills its limit to the
+// last byte with the single counter's 256 bytes fits as before.
+constexpr size_t kQueueRoom = kCounterBytes;
 int launch_batched(const SicView *views, int cpd, int softening, const PairConst &pc, const TileShape &ts,
                    const WorkItem *items, int32_t nitems, const QueueClear &qc, bool cleared, void *stream);
 // Bounding boxes follow a padded source stream of nsrc_blocks blocks.

@@ -503,7 +503,7 @@ void task_rows(const Task &t, uint64_t *r0, uint64_t *r1) {
 
 // Device bytes a SIC adds to a group (plan + work + host-mode slabs).
 size_t task_bytes(const nf_sic &s, int path, int32_t n_chunks) {
-    size_t b = plan_layout(s, 0, n_chunks).total + work_layout(s, path, 0).total + sizeof(SicView) + kCounterBytes;
+    size_t b = plan_layout(s, 0, n_chunks).total + work_layout(s, path, 0).total + sizeof(SicView) + 256;
     b += ((size_t)s.NSinkBlocks + 2 * (size_t)s.NSinkSets) * sizeof(WorkItem);  // at most one item per block + tails
     if (s.mem == NF_MEM_HOST) {
         for (int c = 0; c < s.nfwidth; c++) b += align_up(12 * (size_t)s.Nslab[c], 256);
@@ -1264,8 +1264,9 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
             }
         }
     }
-    if (plan_total + work_total + slab_total > rt.max_buffer_bytes)
-        return fail(NF_ERR_CAPACITY, "SIC group needs " + std::to_string(plan_total + work_total + slab_total) +
+    const size_t need = plan_total + work_total + slab_total - kQueueRoom;
+    if (need > rt.max_buffer_bytes)
+        return fail(NF_ERR_CAPACITY, "SIC group needs " + std::to_string(need) +
                                          " device bytes, buffer holds " + std::to_string(rt.max_buffer_bytes));
     if ((rc = w.plan.ensure(plan_total)) || (rc = w.work.ensure(work_total)) || (rc = w.pin_census.ensure(32)) ||
         (rc = w.pin_plan.ensure(dplan ? head : plan_total)))
@@ -1768,7 +1769,8 @@ void worker_main(Runtime *rt, Worker *w) {
             rt->inflight++;
             uint64_t work = queued_interactions(*g[0]);
             while (path == NF_PATH_BATCHED && (int)g.size() < limit && work < rt->group_interactions &&
-                   (g[0]->dp.on || work < kHostGroupWork || g.size() < share) && !rt->queue.empty() && rt->queue.front()->dp.on == g[0]->dp.on &&
+                   (g[0]->dp.on || work < kHostGroupWork || g.size() < share) && !rt->queue.empty() &&
+                   rt->queue.front()->dp.on == g[0]->dp.on &&
                    compatible(g[0]->sic, rt->queue.front()->sic)) {
                 const size_t b = queued_bytes(*rt->queue.front(), path);
                 if (bytes + b > rt->max_buffer_bytes) break;
@@ -2343,7 +2345,7 @@ namespace {
 // first use on it until the process ends.  In host code `scratch` names a
 // host-side stand-in, never the device memory: kernels, copies and fills
 // take the address hipGetSymbolAddress gives for the current device.
-__device__ __align__(256) char scratch[NF_NOALLOC_SCRATCH_BYTES];
+__device__ __align__(256) char scratch[NF_NOALLOC_SCRATCH_BYTES + kQueueRoom];
 
 constexpr int kNoallocMaxDevices = 64;
 char *g_noalloc_dev[kNoallocMaxDevices];  // per device: the address of `scratch` there
@@ -2351,7 +2353,7 @@ char *g_noalloc_dev[kNoallocMaxDevices];  // per device: the address of `scratch
 // Host image of the upload (view, work list, plan arrays) and the counting
 // sort's cursors, static so that a call allocates no host memory either.
 constexpr size_t kNoallocHostBytes = 32u << 20;
-alignas(256) char g_noalloc_host[kNoallocHostBytes];
+alignas(256) char g_noalloc_host[kNoallocHostBytes + kQueueRoom];
 uint32_t g_noalloc_cursor[2 * kItemBuckets + 1];
 
 // Calls share the scratch of their GPU and the host image: one at a time.
@@ -2364,6 +2366,9 @@ struct NoallocLayout {
     size_t items_max;
     PlanLayout plan;
     WorkLayout work;
+    // Of the limits' bytes (the arrays hold kQueueRoom more).
+    size_t image_need() const { return image - kQueueRoom; }
+    size_t need() const { return total - kQueueRoom; }
 };
 
 NoallocLayout noalloc_layout(const nf_sic &s, bool y_planes) {
@@ -2411,16 +2416,16 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     // Tiles are split over the source pencils where that fits the scratch too.
     uint64_t y_cost = y_split_cost(s.DirectTotal, true);
     NoallocLayout L = noalloc_layout(s, y_cost != UINT64_MAX);
-    if (y_cost != UINT64_MAX && (L.total > NF_NOALLOC_SCRATCH_BYTES || L.image > kNoallocHostBytes)) {
+    if (y_cost != UINT64_MAX && (L.need() > NF_NOALLOC_SCRATCH_BYTES || L.image_need() > kNoallocHostBytes)) {
         y_cost = UINT64_MAX;
         L = noalloc_layout(s, false);
     }
-    if (L.total > NF_NOALLOC_SCRATCH_BYTES)
-        return fail(NF_ERR_CAPACITY, "SIC needs " + std::to_string(L.total) + " bytes of device scratch; "
+    if (L.need() > NF_NOALLOC_SCRATCH_BYTES)
+        return fail(NF_ERR_CAPACITY, "SIC needs " + std::to_string(L.need()) + " bytes of device scratch; "
                                      "nf_execute_sic_noalloc holds " + std::to_string((uint64_t)NF_NOALLOC_SCRATCH_BYTES) +
                                      " (split the slab's rows into smaller SICs)");
-    if (L.image > kNoallocHostBytes)
-        return fail(NF_ERR_CAPACITY, "SIC plan image of " + std::to_string(L.image) + " bytes exceeds the " +
+    if (L.image_need() > kNoallocHostBytes)
+        return fail(NF_ERR_CAPACITY, "SIC plan image of " + std::to_string(L.image_need()) + " bytes exceeds the " +
                                          std::to_string((uint64_t)kNoallocHostBytes) + "-byte host image");
 
     std::lock_guard<std::mutex> lk(g_noalloc_m);
