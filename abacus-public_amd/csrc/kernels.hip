@@ -11,7 +11,7 @@
 //       reference's pair forms (DirectGPUKernels.cuh) and BLOCK_ACCUM tiles.
 //   k_coadd_plain  FP32 co-add of the W partials per sink in the reference's
 //       k order (PencilPlan.cc:140-207 as driven by PencilTask.cu:237-247).
-//   k_batched    persistent kernel draining a work queue sorted by cost;
+//   k_batched    persistent kernel draining work queues dealt from a list sorted by cost;
 //       FP32 tile sums accumulated into FP64 per-pencil partials.
 //   k_coadd_f64  FP64 reduction of the W partials per sink.
 //

@@ -203,7 +203,7 @@ typedef struct nf_setup_params {
     int32_t use_pinned;           /* UsePinnedGPUMemory: -1 auto, 0 no, 1 yes */
     int32_t path;                 /* nf_path used by nf_submit */
     int32_t sinks_per_lane;       /* batched path register tile: 1, 2 or 4 (0: auto) */
-    int32_t source_tile;          /* batched path TwoSum tile depth (0: auto) */
+    int32_t source_tile;          /* batched path source tile depth (0: auto) */
     int32_t gpu_streams;          /* HIP streams the workers enqueue on: 0 one per
                                      worker; 1 one shared stream (tasks run back to
                                      back on the GPU while the workers still prepare
@@ -311,8 +311,9 @@ int nf_get_throughput(nf_throughput *out);
  * sink-pencil occupancies (the share of its sinks in pencils of <64, 64-255,
  * 256-1023 and >=1024 sinks, in quarters) and on its size class (<2^31,
  * <2^33 or more pair interactions); the first group with a new key times each
- * candidate shape on its own launch and the fastest is kept for every later
- * group with that key.  Every shape gives bitwise the same accelerations.
+ * candidate shape on its own launch.  Every later group with that key takes
+ * 2 sinks per lane and 4 waves, or whichever was clearly faster (by 2% and by
+ * 15 us).  Every shape gives bitwise the same accelerations.
  * Writes the table as JSON into buf; returns the length it needs (excluding
  * the terminator), or < 0. */
 int nf_autotune_table(char *buf, size_t len);
