@@ -1010,8 +1010,8 @@ __device__ __forceinline__ void pair_box(float sx, float sy, float sz, float kx,
 struct Sources4 {
     float4 s[4];
     __device__ __forceinline__ void load(const NF_CONST float4 *p) {
-        typedef float Float16 __attribute__((ext_vector_type(16)));
-        const Float16 v = *(const NF_CONST Float16 *)p;
+        typedef float F32x16 __attribute__((ext_vector_type(16)));
+        const F32x16 v = *(const NF_CONST F32x16 *)p;
 #pragma unroll
         for (int i = 0; i < 4; i++) s[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], 0.f);
     }

@@ -73,3 +73,29 @@ def test_plain_pair_pieces_vs_fp64(softening):
             tol = 2 * 4 * 3 * 0.36 * 2.0 ** -25 / (0.3 * 0.004) + 10 * 50 * 2.0 ** -24
             assert rel_err(acc, ref).max() <= tol
             assert np.abs(acc[:, 3] - ref[:, 3]).max() <= 1e-5 * float(b2) * len(U)
+
+
+@pytest.mark.parametrize("path,s", [("plain", 0), ("batched", 1), ("batched", 2), ("batched", 4)])
+def test_source_counts_vs_fp64(path, s):
+    """Lone cells around the tile loop's source batches and the blocks' ends
+    (16, 64), each in a pencil whose other cells are empty."""
+    cpd, soft, counts = 9, 0.03, (1, 15, 16, 17, 48, 63, 64, 65, 80)
+    rng = np.random.default_rng(16)
+    pos = [synth.cell_centre(np.array([4, 3 * (i // 3), 3 * (i % 3)]), cpd) + (rng.random((n, 3)) - 0.5) * (0.9 / cpd)
+           for i, n in enumerate(counts)]
+    box = synth.box_from_global(np.concatenate(pos), cpd)
+    eps, e = synth.eps_param("single_spline", soft)
+    b2 = synth.fof_b2(0.1)
+    with nfm.NearFieldDriver(cpd, soft, b2, softening="single_spline", path=path, buffers_per_device=1,
+                             max_buffer_bytes=1 << 30, **({"sinks_per_lane": s} if s else {})) as drv:
+        acc = np.full((box.slab(4).n, 4), np.nan, np.float32)
+        drv.execute_slab(box, 4, acc, blocking=True)
+        drv.finalize(4)
+    sl, ix, ce = po.slab_sinks(box, 4)
+    ref = po.direct_f64(box, R, "single_spline", eps, b2, sl, ix, ce)
+    # Per source, in the output's units (e^3 a): the force's slope is at most 10, a separation
+    # is off by 3 roundings of coordinates of at most 0.36, and ten more roundings of a term of
+    # at most 2.5 e; the plain path's FLOAT cell offsets double the first.
+    tol = max(counts) * (2 * 10 * 3 ** 0.5 * 3 * 0.36 * 2.0 ** -25 + 10 * 2.0 ** -24 * 2.5 * e)
+    assert np.abs(acc[:, :3] - ref[:, :3]).max() <= tol
+    assert np.abs(acc[:, 3] - ref[:, 3]).max() <= 1e-5 * float(b2) * max(counts)
