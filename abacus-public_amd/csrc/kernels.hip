@@ -1515,6 +1515,10 @@ __device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, 
             }
         }
     }
+    // The last block's reads come before whatever the wave's next item writes
+    // there: full_item's sums are doubles, which the compiler may take for
+    // other memory than these float4.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     for (int m = G; m > 1;) {  // groups [half, m) onto [0, m - half)
         const int half = (m + 1) / 2;
 #pragma unroll
