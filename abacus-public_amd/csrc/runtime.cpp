@@ -118,6 +118,7 @@ struct DevBuf {
         const size_t want = bytes + bytes / 4 + (1 << 20);
         hipError_t e = hipMalloc(&p, want);
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // (the next launch would report it)
             p = nullptr;
             return fail(NF_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
         }
@@ -142,6 +143,7 @@ struct PinBuf {
         const size_t want = bytes + bytes / 4 + (1 << 20);
         hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             p = nullptr;
             return fail(NF_ERR_NOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
         }
@@ -1011,7 +1013,7 @@ GPlanScratch gplan_scratch(const std::vector<Task *> &g) {
 // cellinfo slabs go up through the slab cache (held in `cslot` until the
 // group is done) and the counting kernels are enqueued on the planning
 // stream.  Nothing waits for them: each SIC is laid out for the bounds of
-// its sizes (dp_bounds, set here), the kernels that follow read phase A's
+// its sizes (dp_bounds, set before), the kernels that follow read phase A's
 // counts from device memory, and the totals come back with the group's
 // results.  Fills in[i] for phase B.
 int plan_phase_a(Runtime &rt, Worker &w, std::vector<Task *> &g, std::vector<Runtime::Slot *> &cslot,
@@ -1031,7 +1033,6 @@ int plan_phase_a(Runtime &rt, Worker &w, std::vector<Task *> &g, std::vector<Run
     for (size_t i = 0; i < n; i++) {
         Task &t = *g[i];
         nf_sic &s = t.sic;
-        dp_bounds(s, &t.dp.chunks_bound, &t.dp.items_bound);
         if (y_cost != UINT64_MAX) t.dp.items_bound = y_items_bound(s);
         GPlanIn &gi = in[i];
         gi.y_cost = y_cost;
@@ -1085,23 +1086,64 @@ int apply_group_totals(Worker &w, std::vector<Task *> &g) {
     return rc;
 }
 
+// Where a group's plan upload and working set lie.  Plan upload: [views][group
+// SICs][first waves][items][counter][plan arrays of each SIC]; a device-planned
+// group uploads the head (up to the items) only.
+struct GroupLayout {
+    size_t o_gsic = 0, o_gfirst = 0, head = 0;  // o_gfirst: gather, then co-add
+    size_t o_counter = 0, plan_total = 0, work_total = 0;
+    std::vector<size_t> o_itemset;
+    std::vector<PlanLayout> plan;
+    std::vector<WorkLayout> work;
+};
+// nitems: the lengths of its work lists, or their bounds; planes: tiles may be
+// split over the source pencils.
+GroupLayout group_layout(const std::vector<Task *> &g, int path, const std::vector<size_t> &nitems, bool planes) {
+    GroupLayout L;
+    const size_t n = g.size();
+    L.o_gsic = align_up(sizeof(SicView) * n, 64);
+    L.o_gfirst = align_up(L.o_gsic + sizeof(GroupSic) * n, 64);
+    L.head = align_up(L.o_gfirst + 2 * sizeof(int32_t) * (n + 1), 256);
+    size_t o = L.head;
+    for (size_t m : nitems) {
+        L.o_itemset.push_back(o);
+        o += align_up(sizeof(WorkItem) * std::max<size_t>(m, 1), 256);
+    }
+    L.o_counter = std::max(o, L.head + 256);
+    L.plan_total = align_up(L.o_counter + kCounterBytes, 256);
+    for (const Task *t : g) {
+        L.plan.push_back(plan_layout(t->sic, L.plan_total,
+                                     t->dp.on ? (int32_t)t->dp.chunks_bound : count_coadd_chunks(t->sic)));
+        L.plan_total += L.plan.back().total;
+        L.work.push_back(work_layout(t->sic, path, L.work_total, planes ? t->sic.nfwidth : 1));
+        L.work_total += L.work.back().total;
+    }
+    return L;
+}
+// Of the buffer's limit; slabs: the device slabs the group holds beside it.
+size_t group_need(const GroupLayout &L, size_t slabs) { return L.plan_total + L.work_total + slabs - kQueueRoom; }
+
 // The y_cost of a group's launch: UINT64_MAX (no tile is split over the source
-// pencils, the partials have one plane) unless the launch is small, and its
-// planes and its longer work list fit the buffer.
+// pencils, the partials have one plane) unless the launch is small.
 uint64_t group_y_cost(const Runtime &rt, const std::vector<Task *> &g) {
     if (rt.params.path != NF_PATH_BATCHED) return UINT64_MAX;
-    uint64_t work = 0, planes = 0, bytes = 0;
+    uint64_t work = 0, planes = 0;
     for (const Task *t : g) work += queued_interactions(*t);
     const uint64_t cost = y_split_cost(work, !g[0]->dp.on);
     if (cost == UINT64_MAX) return cost;
-    for (const Task *t : g) {
-        nf_sic s = t->sic;
-        uint64_t chunks, items;
-        if (t->dp.on) dp_bounds(s, &chunks, &items);
-        planes += y_plane_bytes((uint64_t)s.NSinkBlocks, s.nfwidth);
-        bytes += queued_bytes(*t, rt.params.path) + sizeof(WorkItem) * 3 * y_items_bound(s);  // (3: a trial's lists)
-    }
-    return planes <= kYSplitBytes && bytes + planes <= rt.max_buffer_bytes ? cost : UINT64_MAX;
+    for (const Task *t : g) planes += y_plane_bytes((uint64_t)t->sic.NSinkBlocks, t->sic.nfwidth);
+    return planes <= kYSplitBytes ? cost : UINT64_MAX;
+}
+// Whether a device-planned group (its sizes at their bounds) has room for the
+// planes and for every work list a launch of it may need: reserved before
+// phase A, which counts the items of the one choice.
+bool reserve_planes(const Runtime &rt, Worker &w, const std::vector<Task *> &g, size_t slabs) {
+    size_t items = 0;
+    for (const Task *t : g) items += (size_t)y_items_bound(t->sic);
+    const GroupLayout L =
+        group_layout(g, rt.params.path, std::vector<size_t>(rt.autotune ? 3 : 1, items), true);
+    return group_need(L, slabs) <= rt.max_buffer_bytes && w.plan.ensure(L.plan_total) == NF_OK &&
+           w.work.ensure(L.work_total) == NF_OK;
 }
 
 // Execute a group of compatible SICs on worker w: one plan upload, a gather
@@ -1126,10 +1168,37 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     std::vector<Runtime::Slot *> cslot;
     SlotRelease cell_release{rt, cslot};
     uint64_t cell_bytes = 0;
-    const uint64_t y_cost = group_y_cost(rt, g);
-    if (dplan) {
-        for (Task *t : g)
+    const nf_sic &s0 = g[0]->sic;
+    // Host mode: every distinct host slab of the group once (through the
+    // slab cache), plus a device acceleration slab per SIC.
+    std::vector<const float *> hslab;
+    std::vector<uint64_t> hslab_n;
+    std::vector<size_t> acc_off(n, 0), near_off(n, 0);
+    size_t slab_total = 0;
+    if (s0.mem == NF_MEM_HOST) {
+        for (int i = 0; i < n; i++) {
+            const nf_sic &s = g[i]->sic;
+            for (int c = 0; c < s.nfwidth; c++) {
+                if (std::find(hslab.begin(), hslab.end(), s.SourcePosSlab[c]) != hslab.end()) continue;
+                hslab.push_back(s.SourcePosSlab[c]);
+                hslab_n.push_back(s.Nslab[c]);
+            }
+            acc_off[i] = slab_total;
+            slab_total = align_up(slab_total + 16 * (size_t)s.Nslab[s.nfradius], 256);
+            if (s.kick && s.kick->NearAccOut) {  // and one for the near-field record
+                near_off[i] = slab_total;
+                slab_total = align_up(slab_total + 16 * (size_t)s.Nslab[s.nfradius], 256);
+            }
+        }
+    }
+    if (dplan)
+        for (Task *t : g) {
             if (!t->dp.on) return fail(NF_ERR_STATE, "device-planned and host-planned SICs in one group");
+            dp_bounds(t->sic, &t->dp.chunks_bound, &t->dp.items_bound);
+        }
+    uint64_t y_cost = group_y_cost(rt, g);
+    if (dplan) {
+        if (y_cost != UINT64_MAX && !reserve_planes(rt, w, g, slab_total)) y_cost = UINT64_MAX;
         gs = gplan_scratch(g);
         const int rc = plan_phase_a(rt, w, g, cslot, gin, gs, y_cost, &cell_bytes);
         if (rc) return rc;
@@ -1153,7 +1222,6 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
             trial = true;
         }
     }
-    const nf_sic &s0 = g[0]->sic;
     PairConst pc;
     int rc = derive_pair_const(s0.softening, s0.eps, s0.b2, &pc);
     if (rc) return rc;
@@ -1189,89 +1257,43 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
                 if (std::find(Svals.begin(), Svals.end(), c.sinks_per_lane) == Svals.end()) Svals.push_back(c.sinks_per_lane);
         if (std::find(Svals.begin(), Svals.end(), ts.sinks_per_lane) == Svals.end()) Svals.push_back(ts.sinks_per_lane);
     }
-    // (A device-planned SIC's lists are written on the device; phase A
-    // counted their items.)
-    std::vector<const std::vector<WorkItem> *> itemsets;
-    std::vector<size_t> nitems;
-    for (int S : Svals) {
-        std::vector<WorkItem> &list = w.items[S == 1 ? 0 : S == 2 ? 1 : 2];
-        list.clear();
-        if (!dplan) make_items(S, list);
-        itemsets.push_back(&list);
-        size_t m = list.size();
-        if (dplan)
-            for (Task *t : g) m += (size_t)t->dp.items_bound;
-        nitems.push_back(m);
-    }
     auto items_of = [&](int S) -> int {
         for (size_t k = 0; k < Svals.size(); k++)
             if (Svals[k] == S) return (int)k;
         return 0;
     };
-    size_t items_total = 0;
-    for (size_t v : nitems) items_total += align_up(sizeof(WorkItem) * std::max<size_t>(v, 1), 256);
-
-    // Plan upload: [views][group SICs][first waves][items][counter][plan
-    // arrays of each SIC]; a device-planned group uploads the head (up to the
-    // items) only.
-    const size_t o_views = 0;
-    const size_t o_gsic = align_up(o_views + sizeof(SicView) * (size_t)n, 64);
-    const size_t o_gfirst = align_up(o_gsic + sizeof(GroupSic) * (size_t)n, 64);  // gather, then co-add
-    const size_t head = align_up(o_gfirst + 2 * sizeof(int32_t) * (size_t)(n + 1), 256);
-    const size_t o_items = head;
-    std::vector<size_t> o_itemset(itemsets.size());
-    {
-        size_t o = o_items;
-        for (size_t k = 0; k < itemsets.size(); k++) {
-            o_itemset[k] = o;
-            o += align_up(sizeof(WorkItem) * std::max<size_t>(nitems[k], 1), 256);
+    // The lists, the layout and the memory.  A host-planned group whose planes
+    // or longer lists find no room is laid out again with whole tiles.  (A
+    // device-planned SIC's lists are written on the device; phase A counted
+    // their items.)
+    std::vector<const std::vector<WorkItem> *> itemsets;
+    std::vector<size_t> nitems;
+    GroupLayout L;
+    for (;; y_cost = UINT64_MAX) {
+        itemsets.clear();
+        nitems.clear();
+        for (int S : Svals) {
+            std::vector<WorkItem> &list = w.items[S == 1 ? 0 : S == 2 ? 1 : 2];
+            list.clear();
+            if (!dplan) make_items(S, list);
+            itemsets.push_back(&list);
+            size_t m = list.size();
+            if (dplan)
+                for (Task *t : g) m += (size_t)t->dp.items_bound;
+            nitems.push_back(m);
         }
+        L = group_layout(g, path, nitems, y_cost != UINT64_MAX);
+        const size_t need = group_need(L, slab_total);
+        if (need > rt.max_buffer_bytes)
+            rc = fail(NF_ERR_CAPACITY, "SIC group needs " + std::to_string(need) + " device bytes, buffer holds " +
+                                           std::to_string(rt.max_buffer_bytes));
+        else if (!(rc = w.plan.ensure(L.plan_total)) && !(rc = w.work.ensure(L.work_total)) &&
+                 !(rc = w.pin_census.ensure(32)) && !(rc = w.pin_plan.ensure(dplan ? L.head : L.plan_total)) &&
+                 s0.mem == NF_MEM_HOST)
+            rc = w.slabs.ensure(slab_total);
+        if (rc == NF_OK) break;
+        if (dplan || y_cost == UINT64_MAX) return rc;
     }
-    const size_t o_counter = align_up(o_items + std::max<size_t>(items_total, 256), 256);
-    size_t plan_total = align_up(o_counter + kCounterBytes, 256);
-    std::vector<PlanLayout> PL(n);
-    for (int i = 0; i < n; i++) {
-        PL[i] = plan_layout(g[i]->sic, plan_total,
-                            g[i]->dp.on ? (int32_t)g[i]->dp.chunks_bound : count_coadd_chunks(g[i]->sic));
-        plan_total += PL[i].total;
-    }
-    // Device working set of each SIC.
-    std::vector<WorkLayout> WL(n);
-    size_t work_total = 0;
-    for (int i = 0; i < n; i++) {
-        WL[i] = work_layout(g[i]->sic, path, work_total, y_cost == UINT64_MAX ? 1 : g[i]->sic.nfwidth);
-        work_total += WL[i].total;
-    }
-    // Host mode: every distinct host slab of the group once (through the
-    // slab cache), plus a device acceleration slab per SIC.
-    std::vector<const float *> hslab;
-    std::vector<uint64_t> hslab_n;
-    std::vector<size_t> acc_off(n, 0), near_off(n, 0);
-    size_t slab_total = 0;
-    if (s0.mem == NF_MEM_HOST) {
-        for (int i = 0; i < n; i++) {
-            const nf_sic &s = g[i]->sic;
-            for (int c = 0; c < s.nfwidth; c++) {
-                if (std::find(hslab.begin(), hslab.end(), s.SourcePosSlab[c]) != hslab.end()) continue;
-                hslab.push_back(s.SourcePosSlab[c]);
-                hslab_n.push_back(s.Nslab[c]);
-            }
-            acc_off[i] = slab_total;
-            slab_total = align_up(slab_total + 16 * (size_t)s.Nslab[s.nfradius], 256);
-            if (s.kick && s.kick->NearAccOut) {  // and one for the near-field record
-                near_off[i] = slab_total;
-                slab_total = align_up(slab_total + 16 * (size_t)s.Nslab[s.nfradius], 256);
-            }
-        }
-    }
-    const size_t need = plan_total + work_total + slab_total - kQueueRoom;
-    if (need > rt.max_buffer_bytes)
-        return fail(NF_ERR_CAPACITY, "SIC group needs " + std::to_string(need) +
-                                         " device bytes, buffer holds " + std::to_string(rt.max_buffer_bytes));
-    if ((rc = w.plan.ensure(plan_total)) || (rc = w.work.ensure(work_total)) || (rc = w.pin_census.ensure(32)) ||
-        (rc = w.pin_plan.ensure(dplan ? head : plan_total)))
-        return rc;
-    if (s0.mem == NF_MEM_HOST && (rc = w.slabs.ensure(slab_total))) return rc;
 
     // Slabs: HBM copies through the cache (uploads overlap other groups' kernels).
     std::vector<Runtime::Slot *> hslot(hslab.size(), nullptr);
@@ -1295,14 +1317,14 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     std::vector<DevSlabs> slabs(n);
     std::vector<KickArgs> kicks(n);
     std::vector<float *> accd(n);
-    SicView *views = reinterpret_cast<SicView *>(hp + o_views);
+    SicView *views = reinterpret_cast<SicView *>(hp);
     for (int i = 0; i < n; i++) {
         const nf_sic &s = g[i]->sic;
-        const PlanLayout &L = PL[i];
-        if (!g[i]->dp.on) fill_plan_image(s, L, hp);  // host-planned: copy the arrays, derive the lists
+        const PlanLayout &PL = L.plan[i];
+        if (!g[i]->dp.on) fill_plan_image(s, PL, hp);  // host-planned: copy the arrays, derive the lists
 
         DevPlan &pl = plans[i];
-        pl = dev_plan(s, L, pd);
+        pl = dev_plan(s, PL, pd);
         pl.y_cost = y_cost;
         pl.y_plane = y_cost == UINT64_MAX ? 0 : (int64_t)s.NSinkBlocks * NF_BLOCK_SIZE * 4;
         if (dplan) {  // the actual counts, in device memory; the group's bad cells
@@ -1334,7 +1356,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
             ka.rescale = (float)s.kick->rescale;
             ka.inv_eps3 = (float)s.kick->inv_eps3;
             ka.density_rad2 = s.kick->density_rad2;
-            ka.far = s.mem == NF_MEM_HOST ? reinterpret_cast<const float *>(wb + WL[i].o_far) : s.kick->FarAccSlab;
+            ka.far = s.mem == NF_MEM_HOST ? reinterpret_cast<const float *>(wb + L.work[i].o_far) : s.kick->FarAccSlab;
             if (s.kick->NearAccOut)
                 ka.near_out = s.mem == NF_MEM_HOST ? reinterpret_cast<float *>(db + near_off[i]) : s.kick->NearAccOut;
             ka.far_base = s.mem == NF_MEM_HOST ? (int64_t)r0 : 0;
@@ -1350,16 +1372,16 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         v.sink_slab = sl.pos[s.nfradius];
         v.sink_n = s.Nslab[s.nfradius];
         v.aos = sl.aos;
-        v.sources4 = wb + WL[i].o_src;
-        v.box4 = box_after(wb + WL[i].o_src, s.NSourceBlocks);
-        v.partial = reinterpret_cast<double *>(wb + WL[i].o_part);
+        v.sources4 = wb + L.work[i].o_src;
+        v.box4 = box_after(wb + L.work[i].o_src, s.NSourceBlocks);
+        v.partial = reinterpret_cast<double *>(wb + L.work[i].o_part);
         v.y_plane = pl.y_plane;
         v.W = s.nfwidth;
         v.R = s.nfradius;
     }
     // The group-wide gather and co-add launches' view of each SIC.
-    GroupSic *gsic = reinterpret_cast<GroupSic *>(hp + o_gsic);
-    int32_t *gfirst = reinterpret_cast<int32_t *>(hp + o_gfirst), *cfirst = gfirst + (n + 1);
+    GroupSic *gsic = reinterpret_cast<GroupSic *>(hp + L.o_gsic);
+    int32_t *gfirst = reinterpret_cast<int32_t *>(hp + L.o_gfirst), *cfirst = gfirst + (n + 1);
     gfirst[0] = cfirst[0] = 0;
     uint64_t sinks = 0, cells = 0;
     for (Task *t : g) {
@@ -1375,8 +1397,8 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         G.pl = plans[i];
         G.sl = slabs[i];
         G.kick = kicks[i];
-        G.sources4 = wb + WL[i].o_src;
-        G.partial = wb + WL[i].o_part;
+        G.sources4 = wb + L.work[i].o_src;
+        G.partial = wb + L.work[i].o_part;
         G.acc4 = accd[i];
         G.out_scale = pc.out_scale;
         gfirst[i + 1] = gfirst[i] + group_gather_waves(plans[i]);
@@ -1384,23 +1406,23 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     }
     for (size_t k = 0; k < itemsets.size(); k++)
         if (!itemsets[k]->empty())
-            std::memcpy(hp + o_itemset[k], itemsets[k]->data(), sizeof(WorkItem) * itemsets[k]->size());
+            std::memcpy(hp + L.o_itemset[k], itemsets[k]->data(), sizeof(WorkItem) * itemsets[k]->size());
     const auto t_fill = clk::now();
     // The plan image goes up on the copy stream, overlapping the kernels of
     // the group before (this worker's previous group has completed, so its
     // plan buffer is free).  A device-planned SIC's image is its view only;
     // phase B and the work lists fill the rest on the planning stream.
     if (dplan) {
-        NF_HIP(hipMemcpyAsync(w.plan.p, hp, head, hipMemcpyHostToDevice, w.pstream));
+        NF_HIP(hipMemcpyAsync(w.plan.p, hp, L.head, hipMemcpyHostToDevice, w.pstream));
         char *sc = static_cast<char *>(w.gscratch.p);
         int32_t *shared = reinterpret_cast<int32_t *>(sc + gs.o_shared);
         std::vector<GPlanOut> go(n);
         for (int i = 0; i < n; i++) {
-            go[i] = plan_out(pd, PL[i], i, shared, reinterpret_cast<int32_t *>(sc + gs.o_part[i]));
+            go[i] = plan_out(pd, L.plan[i], i, shared, reinterpret_cast<int32_t *>(sc + gs.o_part[i]));
             go[i].group = shared;
             for (size_t k = 0; k < Svals.size(); k++) {
                 const int ti = Svals[k] == 1 ? 0 : Svals[k] == 2 ? 1 : 2;
-                go[i].items[ti] = reinterpret_cast<WorkItem *>(pd + o_itemset[k]);
+                go[i].items[ti] = reinterpret_cast<WorkItem *>(pd + L.o_itemset[k]);
             }
         }
         char *pg = static_cast<char *>(w.pin_gplan.p);
@@ -1423,7 +1445,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         if (e) return fail(NF_ERR_HIP, std::string("device plan launch: ") + hipGetErrorString((hipError_t)e));
         NF_HIP(hipEventRecord(w.gplan_ready, w.pstream));
     } else {
-        NF_HIP(hipMemcpyAsync(w.plan.p, hp, plan_total, hipMemcpyHostToDevice, rt.cache.up));
+        NF_HIP(hipMemcpyAsync(w.plan.p, hp, L.plan_total, hipMemcpyHostToDevice, rt.cache.up));
     }
     // Host mode with a fused kick: the far-field accelerations of the sink
     // rows go up beside the plan (pinned ones directly, else through staging).
@@ -1450,7 +1472,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
                 par_memcpy(static_cast<char *>(w.pin_far.p) + off, src, nb);
                 src = reinterpret_cast<const float *>(static_cast<char *>(w.pin_far.p) + off);
             }
-            NF_HIP(hipMemcpyAsync(wb + WL[i].o_far, src, nb, hipMemcpyHostToDevice, rt.cache.up));
+            NF_HIP(hipMemcpyAsync(wb + L.work[i].o_far, src, nb, hipMemcpyHostToDevice, rt.cache.up));
             off += nb;
         }
     }
@@ -1460,7 +1482,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     hipStream_t stream = rt.shared ? rt.shared : w.stream;
     std::unique_lock<std::mutex> enqueue_lock(rt.enqueue, std::defer_lock);
     if (rt.shared) enqueue_lock.lock();
-    uint64_t to_dev = (dplan ? sizeof(SicView) * (size_t)n : plan_total) + far_bytes + cell_bytes, from_dev = 0;
+    uint64_t to_dev = (dplan ? sizeof(SicView) * (size_t)n : L.plan_total) + far_bytes + cell_bytes, from_dev = 0;
     // With graphs, the sequence below is captured and launched as one graph.
     const bool use_graph = rt.params.use_graphs && !trial;
     struct CaptureGuard {  // ends an open capture on every early return
@@ -1489,15 +1511,16 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         capture.on = true;
     }
     int e = 0;
-    const GroupSic *gsic_d = reinterpret_cast<const GroupSic *>(pd + o_gsic);
-    const int32_t *gfirst_d = reinterpret_cast<const int32_t *>(pd + o_gfirst), *cfirst_d = gfirst_d + (n + 1);
+    const GroupSic *gsic_d = reinterpret_cast<const GroupSic *>(pd + L.o_gsic);
+    const int32_t *gfirst_d = reinterpret_cast<const int32_t *>(pd + L.o_gfirst), *cfirst_d = gfirst_d + (n + 1);
     // The batched launch's queues, cleared by the gather.  A device-planned
     // group's list lengths and bad cells are in its shared planning area.
     const int32_t *gshared =
         dplan ? reinterpret_cast<const int32_t *>(static_cast<char *>(w.gscratch.p) + gs.o_shared) : nullptr;
     auto queues = [&](const TileShape &shape) {
         const int ti = shape.sinks_per_lane == 1 ? 0 : shape.sinks_per_lane == 2 ? 1 : 2;
-        return QueueClear{reinterpret_cast<int32_t *>(pd + o_counter), gshared ? gshared + kPlanGroupItems + ti : nullptr,
+        return QueueClear{reinterpret_cast<int32_t *>(pd + L.o_counter),
+                          gshared ? gshared + kPlanGroupItems + ti : nullptr,
                           gshared ? gshared + kPlanGroupBad : nullptr, rt.params.census ? 1 : 0};
     };
     if (path == NF_PATH_BATCHED) {
@@ -1507,17 +1530,18 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     }
     else
         for (int i = 0; i < n && !e; i++)
-            e = launch_gather(plans[i], slabs[i], false, wb + WL[i].o_sinks, wb + WL[i].o_src, QueueClear{}, stream);
+            e = launch_gather(plans[i], slabs[i], false, wb + L.work[i].o_sinks, wb + L.work[i].o_src, QueueClear{},
+                              stream);
     if (e) return fail(NF_ERR_HIP, std::string("gather launch: ") + hipGetErrorString((hipError_t)e));
     if (!use_graph) NF_HIP(hipEventRecord(w.ev[2], stream));
     std::vector<hipEvent_t> tev;
     unsigned long long *census = nullptr;  // batched path: interactions per pair form (device)
     if (path == NF_PATH_BATCHED) {
         if (rt.params.census)  // in the counter's slot
-            census = reinterpret_cast<unsigned long long *>(pd + o_counter + kCensusBytes);
+            census = reinterpret_cast<unsigned long long *>(pd + L.o_counter + kCensusBytes);
         auto launch = [&](const TileShape &shape) {
-            return launch_batched(reinterpret_cast<const SicView *>(pd + o_views), s0.cpd, s0.softening, pc, shape,
-                                  reinterpret_cast<const WorkItem *>(pd + o_itemset[items_of(shape.sinks_per_lane)]),
+            return launch_batched(reinterpret_cast<const SicView *>(pd), s0.cpd, s0.softening, pc, shape,
+                                  reinterpret_cast<const WorkItem *>(pd + L.o_itemset[items_of(shape.sinks_per_lane)]),
                                   (int32_t)nitems[items_of(shape.sinks_per_lane)], queues(shape),
                                   !trial && gfirst[n] > 0, stream);
         };
@@ -1540,8 +1564,8 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         }
     } else {
         for (int i = 0; i < n && !e; i++)
-            e = launch_plain(plans[i], s0.softening, pc, wb + WL[i].o_sinks, wb + WL[i].o_src, wb + WL[i].o_part,
-                             stream);
+            e = launch_plain(plans[i], s0.softening, pc, wb + L.work[i].o_sinks, wb + L.work[i].o_src,
+                             wb + L.work[i].o_part, stream);
     }
     if (e) return fail(NF_ERR_HIP, std::string("direct kernel launch: ") + hipGetErrorString((hipError_t)e));
     if (!use_graph) NF_HIP(hipEventRecord(w.ev[3], stream));
@@ -1549,7 +1573,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
         e = launch_coadd_group(gsic_d, cfirst_d, n, cfirst[n], clanes, y_cost != UINT64_MAX, stream);
     else
         for (int i = 0; i < n && !e; i++)
-            e = launch_coadd_plain(plans[i], wb + WL[i].o_part, accd[i], kicks[i], clanes, stream);
+            e = launch_coadd_plain(plans[i], wb + L.work[i].o_part, accd[i], kicks[i], clanes, stream);
     if (e) return fail(NF_ERR_HIP, std::string("co-add launch: ") + hipGetErrorString((hipError_t)e));
     if (use_graph) {
         hipGraph_t graph = nullptr;
