@@ -2369,8 +2369,8 @@ extern "C" int nf_stream_end(void) {
 namespace nf {
 namespace {
 
-// Device scratch of nf_execute_sic_noalloc: a SIC's plan image (view, work
-// list, queue counter, plan arrays), its source stream with the block boxes,
+// Device scratch of nf_execute_sic_noalloc: a SIC's plan image (view, plan
+// arrays, work list), its queue counter, its source stream with the block boxes,
 // and its FP64 partials.  Each GPU holds its own copy from the library's
 // first use on it until the process ends.  In host code `scratch` names a
 // host-side stand-in, never the device memory: kernels, copies and fills
@@ -2380,25 +2380,27 @@ __device__ __align__(256) char scratch[NF_NOALLOC_SCRATCH_BYTES + kQueueRoom];
 constexpr int kNoallocMaxDevices = 64;
 char *g_noalloc_dev[kNoallocMaxDevices];  // per device: the address of `scratch` there
 
-// Host image of the upload (view, work list, plan arrays) and the counting
+// Host image of the upload (view, plan arrays, work list) and the counting
 // sort's cursors, static so that a call allocates no host memory either.
 constexpr size_t kNoallocHostBytes = 32u << 20;
-alignas(256) char g_noalloc_host[kNoallocHostBytes + kQueueRoom];
+alignas(256) char g_noalloc_host[kNoallocHostBytes];
 uint32_t g_noalloc_cursor[2 * kItemBuckets + 1];
 
 // Calls share the scratch of their GPU and the host image: one at a time.
 std::mutex g_noalloc_m;
 
-// Where one SIC sits in the scratch: [view][items][counter][plan arrays]
-// (the uploaded image) then [source stream + boxes][partials].
+// Where one SIC sits in the scratch: [view][plan arrays][items] (the host
+// image) then [counter][source stream + boxes][partials].  The list comes last
+// in the image, which is uploaded up to the list's real end: its bound is W
+// items a block (a CPD 45 slab at 55 per cell: 0.8 MB beside 0.4 MB of plan
+// arrays; where few tiles are split, at CPD 129 with 4 per cell, a call takes
+// 0.665 ms, with the bound uploaded 0.711).
 struct NoallocLayout {
     size_t o_items, o_counter, o_plan, image, o_work, total;
     size_t items_max;
     PlanLayout plan;
     WorkLayout work;
-    // Of the limits' bytes (the arrays hold kQueueRoom more).
-    size_t image_need() const { return image - kQueueRoom; }
-    size_t need() const { return total - kQueueRoom; }
+    size_t need() const { return total - kQueueRoom; }  // of the limit's bytes (the scratch holds kQueueRoom more)
 };
 
 NoallocLayout noalloc_layout(const nf_sic &s, bool y_planes) {
@@ -2406,12 +2408,12 @@ NoallocLayout noalloc_layout(const nf_sic &s, bool y_planes) {
     // At most one item per padded sink block (and source pencil, if tiles may
     // be split over them) plus one tail per pencil, whatever the tile split.
     L.items_max = y_planes ? (size_t)y_items_bound(s) : (size_t)s.NSinkBlocks + (size_t)s.NSinkSets;
-    L.o_items = align_up(sizeof(SicView), 256);
-    L.o_counter = align_up(L.o_items + sizeof(WorkItem) * std::max<size_t>(L.items_max, 1), 256);
-    L.o_plan = align_up(L.o_counter + kCounterBytes, 256);
+    L.o_plan = align_up(sizeof(SicView), 256);
     L.plan = plan_layout(s, L.o_plan, count_coadd_chunks(s));
-    L.image = L.o_plan + L.plan.total;
-    L.o_work = align_up(L.image, 256);
+    L.o_items = L.o_plan + L.plan.total;
+    L.image = L.o_items + sizeof(WorkItem) * std::max<size_t>(L.items_max, 1);
+    L.o_counter = align_up(L.image, 256);
+    L.o_work = align_up(L.o_counter + kCounterBytes, 256);
     L.work = work_layout(s, NF_PATH_BATCHED, L.o_work, y_planes ? s.nfwidth : 1);
     L.total = L.o_work + L.work.total;
     return L;
@@ -2446,7 +2448,7 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     // Tiles are split over the source pencils where that fits the scratch too.
     uint64_t y_cost = y_split_cost(s.DirectTotal, true);
     NoallocLayout L = noalloc_layout(s, y_cost != UINT64_MAX);
-    if (y_cost != UINT64_MAX && (L.need() > NF_NOALLOC_SCRATCH_BYTES || L.image_need() > kNoallocHostBytes)) {
+    if (y_cost != UINT64_MAX && (L.need() > NF_NOALLOC_SCRATCH_BYTES || L.image > kNoallocHostBytes)) {
         y_cost = UINT64_MAX;
         L = noalloc_layout(s, false);
     }
@@ -2454,8 +2456,8 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
         return fail(NF_ERR_CAPACITY, "SIC needs " + std::to_string(L.need()) + " bytes of device scratch; "
                                      "nf_execute_sic_noalloc holds " + std::to_string((uint64_t)NF_NOALLOC_SCRATCH_BYTES) +
                                      " (split the slab's rows into smaller SICs)");
-    if (L.image_need() > kNoallocHostBytes)
-        return fail(NF_ERR_CAPACITY, "SIC plan image of " + std::to_string(L.image_need()) + " bytes exceeds the " +
+    if (L.image > kNoallocHostBytes)
+        return fail(NF_ERR_CAPACITY, "SIC plan image of " + std::to_string(L.image) + " bytes exceeds the " +
                                          std::to_string((uint64_t)kNoallocHostBytes) + "-byte host image");
 
     std::lock_guard<std::mutex> lk(g_noalloc_m);
@@ -2521,10 +2523,10 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     v.R = s.nfradius;
 
     // Upload, gather, one persistent launch, co-add, on the caller's stream;
-    // the gather clears the queues.  The
-    // host image stays untouched until the stream has drained.
+    // the gather clears the queues.  The host image stays untouched until the
+    // stream has drained.
     hipStream_t st = static_cast<hipStream_t>(stream);
-    NF_HIP(hipMemcpyAsync(d, h, L.image, hipMemcpyHostToDevice, st));
+    NF_HIP(hipMemcpyAsync(d, h, L.o_items + sizeof(WorkItem) * nitems, hipMemcpyHostToDevice, st));
     const QueueClear qc{reinterpret_cast<int32_t *>(d + L.o_counter), nullptr, nullptr, 0};
     int e = launch_gather(pl, sl, true, nullptr, src, qc, st);
     if (!e)
