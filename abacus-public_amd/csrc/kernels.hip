@@ -526,10 +526,16 @@ __device__ __forceinline__ void clear_queues(const QueueClear &qc, int t) {
     }
 }
 
+// At most 96 SGPRs: above that the segmented form loses a wave per SIMD.  Both
+// forms of the group's gather (below) are faster for it although they spill 6
+// and 90 scalars into VGPR lanes (0 and 32 without the cap): with / without,
+// 512^3 slabs 70.7 / 73.4 us on average, clustered slabs 49.2 / 50.1 us, the
+// segmented gather of one CPD 255 slab 210 / 220 us.  One SIC's: no difference
+// beyond the builds' own (whole pencils 15.8 us, segmented 19.5-20.5 us).
 template <bool SEG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned(DevPlan pl, DevSlabs sl, float4 *__restrict__ out,
-                                                               float4 *__restrict__ box, float cpdf,
-                                                               double invcpd, QueueClear qc) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned(
+    DevPlan pl, DevSlabs sl, float4 *__restrict__ out, float4 *__restrict__ box, float cpdf, double invcpd,
+    QueueClear qc) {
     if (blockIdx.x == 0 && qc.counter) clear_queues(qc, threadIdx.x);
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x / kWave));
     if (w >= gather_waves(pl.nsrc_sets, pl.nsrc_blocks, pl.max_src_blocks) || plan_bad(pl)) return;
@@ -552,9 +558,9 @@ __device__ __forceinline__ int group_sic_of(const int32_t *first, int n, int w) 
 // Every SIC's source gather of a launch group in one launch: a group of
 // small SICs (a clustered box's) fills the GPU where one SIC's pencils do not.
 template <bool SEG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned_group(const GroupSic *__restrict__ g,
-                                                                     const int32_t *__restrict__ first, int n,
-                                                                     float cpdf, double invcpd, QueueClear qc) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(96))) void k_gather_sources_binned_group(
+    const GroupSic *__restrict__ g, const int32_t *__restrict__ first, int n, float cpdf, double invcpd,
+    QueueClear qc) {
     if (blockIdx.x == 0 && qc.counter) clear_queues(qc, threadIdx.x);
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (int)(threadIdx.x / kWave));
     if (w >= cptr<int32_t>(first)[n]) return;

@@ -1754,7 +1754,10 @@ constexpr int kGroupFillWaitUs = 2000;
 // about the time its kernels take, so its SICs are spread over the idle workers
 // once a group holds this many pair interactions (about 1 ms of kernel).  Six
 // SICs of 2e9 went out as groups of 1 and 5, the second 2.6 ms after the first
-// had ended; now as 1, 2, 2 and 1.
+// had ended; now as 1, 2, 2 and 1.  With this line / with group_interactions
+// alone, a pass: 16 SICs of 0.5e9 3.2 / 4.1 ms, eight of 2e9 4.6 / 5.8 ms, a
+// clustered 256^3 box's 9.3 / 11.3 ms, six of 6.7e9 (512^3 slabs) planned before
+// the pass 12.4 / 12.4 ms and planned in it 13.3 / 14.7 ms.
 constexpr uint64_t kHostGroupWork = 3000000000ull;
 
 void worker_main(Runtime *rt, Worker *w) {
