@@ -807,9 +807,12 @@ std::vector<TileShape> tile_candidates(int fixed_s, int fixed_wpw) {
 // of the group's sinks in pencils of <64, 64-255, 256-1023 and >=1024 sinks,
 // in quarters) and the group's size class (below 2^31, below 2^33, or more
 // pair interactions: small launches are limited by their longest items,
-// large ones by throughput).  Coarse on purpose: every new key costs one
-// launch per candidate.
-std::string occupancy_key(const std::vector<Task *> &g) {
+// large ones by throughput), and whether its tiles may be split over the source
+// pencils (split pencils have one-wave tiles whatever the shape, so a split
+// launch says little about a whole one of its size class; the line also differs
+// between lists made on the device and on the host).  Coarse on purpose: every
+// new key costs one launch per candidate.
+std::string occupancy_key(const std::vector<Task *> &g, bool split) {
     double h[4] = {0, 0, 0, 0};
     double tot = 0;
     uint64_t di = 0;
@@ -831,6 +834,7 @@ std::string occupancy_key(const std::vector<Task *> &g) {
     std::ostringstream os;
     for (int b = 0; b < 4; b++) os << (b ? "," : "") << (int)std::lround(4.0 * h[b] / std::max(tot, 1.0));
     os << ";" << (di < (1ull << 31) ? 0 : di < (1ull << 33) ? 1 : 2);
+    os << ";" << (!split ? "whole" : g[0]->dp.on ? "device" : "host");
     return os.str();
 }
 
@@ -1212,7 +1216,7 @@ int run_group(Runtime &rt, Worker &w, std::vector<Task *> &g) {
     std::string tkey;
     bool trial = false;
     if (path == NF_PATH_BATCHED && rt.autotune) {
-        tkey = occupancy_key(g);
+        tkey = occupancy_key(g, y_cost != UINT64_MAX);
         std::lock_guard<std::mutex> lk(rt.tune_m);
         auto it = rt.tune.find(tkey);
         if (it != rt.tune.end()) {
@@ -2327,9 +2331,10 @@ extern "C" int nf_autotune_table(char *buf, size_t len) {
         bool first = true;
         for (const auto &kv : g_rt->tune) {
             const auto &e = kv.second;
-            const size_t semi = kv.first.find(';');
+            const size_t semi = kv.first.find(';'), last = kv.first.rfind(';');
             os << (first ? "" : ",") << "{\"occupancy_quarters\":[" << kv.first.substr(0, semi)
-               << "],\"size_class\":" << kv.first.substr(semi + 1) << ",\"sinks_per_lane\":"
+               << "],\"size_class\":" << kv.first.substr(semi + 1, last - semi - 1) << ",\"split\":\""
+               << kv.first.substr(last + 1) << "\",\"sinks_per_lane\":"
                << e.shape.sinks_per_lane << ",\"waves_per_wg\":" << e.shape.waves_per_wg
                << ",\"waves_per_cu\":" << e.shape.waves_per_cu << ",\"uses\":" << e.uses
                << ",\"interactions\":" << e.interactions << ",\"trial_ms\":[";

@@ -309,8 +309,10 @@ int nf_get_throughput(nf_throughput *out);
  * waves_per_wg fix an axis when nonzero, and the autotuner searches the
  * others.  It keys every launch group on a coarse histogram of its
  * sink-pencil occupancies (the share of its sinks in pencils of <64, 64-255,
- * 256-1023 and >=1024 sinks, in quarters) and on its size class (<2^31,
- * <2^33 or more pair interactions); the first group with a new key times each
+ * 256-1023 and >=1024 sinks, in quarters), on its size class (<2^31,
+ * <2^33 or more pair interactions) and on whether a launch so small splits its
+ * tiles over the source pencils ("whole", or "device" or "host" for lists made
+ * there); the first group with a new key times each
  * candidate shape on its own launch.  Every later group with that key takes
  * 2 sinks per lane and 4 waves, or whichever was clearly faster (by 2% and by
  * 15 us).  Every shape gives bitwise the same accelerations.
