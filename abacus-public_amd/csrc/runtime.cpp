@@ -157,19 +157,6 @@ struct PinBuf {
     }
 };
 
-// A run of like work items of a pencil: tiles of up to `step` sinks from
-// `first` to `end`.  Item i is tile i / ny against source pencil i % ny (ny > 1:
-// kind 3).
-struct ItemRun {
-    int32_t sinkset, first, step, end, kind_sic, ny;
-    int32_t key;  // counting-sort key: the cost's bucket, plus kItemBuckets for a tail
-    int count() const { return (end - first + step - 1) / step * ny; }
-    WorkItem item(int i) const {
-        const int f = first + i / ny * step;
-        return WorkItem{sinkset, f, std::min(step, end - f) + (ny > 1 ? 256 * (i % ny) : 0), kind_sic};
-    }
-};
-
 struct Worker {
     int id = 0;
     int device = 0;
@@ -561,9 +548,7 @@ size_t queued_bytes(const Task &t, int path) {
 }
 uint64_t queued_interactions(const Task &t) { return t.dp.on ? t.dp.interactions : t.sic.DirectTotal; }
 
-// The 1/8-octave bucket of an item's cost (sinks x sources), longest first:
-// bucket 0 holds the most expensive items, kItemBuckets - 1 the cheapest.
-constexpr int kItemBuckets = 1024;
+// The bucket of an item's cost (sinks x sources).
 int cost_bucket(uint64_t cost) {
     if (cost == 0) return kItemBuckets - 1;
     // 8 log2 cost, rounded down: the exponent, and the eighth that the first 8
@@ -661,39 +646,6 @@ void for_each_run(const nf_sic &s, int S, int sic, uint64_t max_tile_cost, uint6
                              kItemBuckets + cost_bucket((uint64_t)(n - tiles) * nsrc)});
         }
 }
-
-// The counting sort of a work list, by cost bucket, of the tiles and of the
-// short tails apart: add() every run, begin(), then place() the same runs in
-// the same order.  A run's items are placed one after the other in its bucket's
-// stretch of its merged run (interleave_pos, stepped without divisions).
-struct ItemSort {
-    uint32_t *start;  // 2 kItemBuckets + 1, zeroed
-    int64_t M = 0, T = 0;
-    void add(const ItemRun &r) { start[r.key + 1] += (uint32_t)r.count(); }
-    size_t begin() {
-        for (int b = 0; b < 2 * kItemBuckets; b++) start[b + 1] += start[b];
-        M = start[kItemBuckets];
-        T = (int64_t)start[2 * kItemBuckets] - M;
-        return (size_t)(M + T);
-    }
-    void place(const ItemRun &r, WorkItem *out) {
-        const int cnt = r.count();
-        const int64_t at = start[r.key];
-        start[r.key] += (uint32_t)cnt;
-        if (r.key >= kItemBuckets) {  // a tail (cnt 1)
-            out[interleave_pos(true, at - M, M, T)] = r.item(0);
-            return;
-        }
-        // tails before tile `at`: at T / M (by a floating division, set right)
-        int64_t before = (int64_t)((double)(at * T) / (double)M), rem = at * T - before * M;
-        if (rem < 0) before--, rem += M;
-        if (rem >= M) before++, rem -= M;
-        for (int i = 0; i < cnt; i++) {
-            out[at + i + before] = r.item(i);
-            for (rem += T; rem >= M; rem -= M) before++;
-        }
-    }
-};
 
 int validate(const nf_sic &s) {
     if (s.nfradius < 0 || s.nfradius > NF_MAX_RADIUS || s.nfwidth != 2 * s.nfradius + 1)

@@ -104,3 +104,20 @@ def test_work_list_interleave_is_an_even_permutation(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=600,
                        env=dict(os.environ, UBSAN_OPTIONS="halt_on_error=1"))
     assert r.returncode == 0 and "even permutation" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
+
+
+def test_work_list_sort_places_every_item(tmp_path):
+    """ItemSort, which places the host's work lists a run at a time (launch
+    groups and the no-allocation entry point), puts every item where a stable
+    sort by cost and interleave_pos put it: tiles, tiles split over the source
+    pencils and short tails, more and fewer tails than tiles, none of either,
+    and launch-group sizes."""
+    if not shutil.which("g++"):
+        pytest.skip("g++ not found")
+    csrc = os.path.join(ROOT, "abacus-public_amd", "csrc")
+    exe = str(tmp_path / "itemsort_check")
+    _run(["g++", "-std=c++17", "-O1", *SAN, "-I", os.path.join(ROOT, "include"), "-I", csrc,
+          os.path.join(ROOT, "tests", "sanitize", "itemsort_check.cpp"), "-o", exe])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=600,
+                       env=dict(os.environ, UBSAN_OPTIONS="halt_on_error=1"))
+    assert r.returncode == 0 and "every item" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
