@@ -62,10 +62,6 @@ __device__ __forceinline__ const NF_CONST T *cptr(const void *p) {
 #define NF_TRANS1(op, a) (void)(a)
 #define NF_TRANS2(op, a, b) (void)(a), (void)(b)
 #endif
-__device__ __forceinline__ float rsq(float x) {
-    NF_TRANS1("v_rsq_f32", x);
-    return x;
-}
 __device__ __forceinline__ float sqrt_(float x) {
     NF_TRANS1("v_sqrt_f32", x);
     return x;
@@ -957,11 +953,6 @@ __device__ __forceinline__ void pair_r2(float sx, float sy, float sz, float kx, 
 }
 // 2. f = 1/r, or r for the cubic Plummer form;
 template <int SOFT>
-__device__ __forceinline__ void pair_f(float &a) {
-    if constexpr (SOFT == NF_SOFT_CUBIC_PLUMMER) NF_TRANS1("v_sqrt_f32", a);
-    else NF_TRANS1("v_rsq_f32", a);
-}
-template <int SOFT>
 __device__ __forceinline__ void pair_f(float &a, float &b) {
     if constexpr (SOFT == NF_SOFT_CUBIC_PLUMMER) NF_TRANS2("v_sqrt_f32", a, b);
     else NF_TRANS2("v_rsq_f32", a, b);
@@ -1002,16 +993,6 @@ __device__ __forceinline__ void pair_sum(float g, float dx, float dy, float dz, 
     az = fmaf(g, dz, az);
 }
 
-template <int SOFT, int MODE>
-__device__ __forceinline__ void pair_box(float sx, float sy, float sz, float kx, float ky, float kz,
-                                         const PairConst &pc, float &ax, float &ay, float &az, float &aw) {
-    float dx, dy, dz, r2;
-    pair_r2<MODE>(sx, sy, sz, kx, ky, kz, pc, dx, dy, dz, r2, aw);
-    float f = r2;
-    pair_f<SOFT>(f);
-    pair_sum(pair_g<SOFT, MODE>(r2, f, pc), dx, dy, dz, ax, ay, az);
-}
-
 // Four sources in scalar registers, by one load.
 struct Sources4 {
     float4 s[4];
@@ -1030,6 +1011,7 @@ __device__ __forceinline__ void pair_group(SrcP sp, const float *kx, const float
                                            const float *kz, const PairConst &pc, float *bx, float *by, float *bz,
                                            float *tw) {
     constexpr int N = P * S;
+    static_assert(N % 2 == 0, "pairs two by two");
     float dx[N], dy[N], dz[N], r2[N], f[N];
 #pragma unroll
     for (int t = 0; t < N; t++) {
@@ -1039,9 +1021,8 @@ __device__ __forceinline__ void pair_group(SrcP sp, const float *kx, const float
         else pair_r2<MHI>(sv.x, sv.y, sv.z, kx[u], ky[u], kz[u], pc, dx[t], dy[t], dz[t], r2[t], tw[u]);
         f[t] = r2[t];
     }
-    if constexpr (N == 1) pair_f<SOFT>(f[0]);
 #pragma unroll
-    for (int t = 0; t + 1 < N; t += 2) pair_f<SOFT>(f[t], f[t + 1]);
+    for (int t = 0; t < N; t += 2) pair_f<SOFT>(f[t], f[t + 1]);
 #pragma unroll
     for (int t = 0; t < N; t++) {
         const int u = t % S;

@@ -198,7 +198,6 @@ struct PairConst {
     float r2add;      // added to r^2 before rsqrt: tau (spline forms) or e^2 (Plummer)
     float b2x;        // density threshold against that r^2: b2 + r2add
     float c1, c2, c3; // single spline, box-unit polynomial (-15 e^-4, 6 e^-5, 10 e^-3); cubic spline: c3 = e^-3
-    float theta;      // tile density sum below which no pair is softened (< 0: none)
     double out_scale; // e^3 for the box-unit spline, 1 otherwise
 };
 
@@ -208,8 +207,6 @@ int derive_pair_const(int softening, float eps, float b2, PairConst *pc);
 // a sink's sum does not depend on which lane, wave or workgroup computes it.
 struct TileShape {
     int sinks_per_lane;   // S: 1, 2 or 4
-    int tile;             // source tile depth
-    int rem_sinks;        // uniform sinks per pass in the remainder path
     int waves_per_cu;     // persistent grid size (0: from occupancy)
     int waves_per_wg;     // workgroup size in waves: 1, 2 or 4 (0: 4)
 };

@@ -53,7 +53,6 @@ int derive_pair_const(int softening, float eps, float b2, PairConst *pc) {
     pc->eps = eps;
     pc->b2 = b2;
     pc->out_scale = 1.0;
-    pc->theta = -1.f;
     if (!(eps > 0.f) || !std::isfinite(eps)) return fail(NF_ERR_INVALID, "eps must be finite and positive");
     if (!(b2 >= 0.f) || !(b2 < 0.5f)) return fail(NF_ERR_INVALID, "b2 must be in [0, 0.5)");
     switch (softening) {
@@ -195,7 +194,7 @@ struct Runtime {
     bool stopping = false;
     int inflight = 0;   // groups taken by workers and not finished (under qm)
     bool warm = false;  // work has been flowing since the queue was last empty (under qm)
-    TileShape shape{2, 64, 4, 0, 4};
+    TileShape shape{2, 0, 4};
     std::vector<TileShape> candidates;  // the autotuner's search (empty: the shape is fixed)
     int max_group = 8;
     uint64_t group_interactions = 12000000000ull;
@@ -751,7 +750,7 @@ std::vector<TileShape> tile_candidates(int fixed_s, int fixed_wpw) {
     std::vector<TileShape> v;
     for (int S : {1, 2, 4})
         for (int wpw : {1, 2, 4})
-            if ((!fixed_s || S == fixed_s) && (!fixed_wpw || wpw == fixed_wpw)) v.push_back(TileShape{S, 64, 4, 0, wpw});
+            if ((!fixed_s || S == fixed_s) && (!fixed_wpw || wpw == fixed_wpw)) v.push_back(TileShape{S, 0, wpw});
     return v;
 }
 
@@ -2490,7 +2489,7 @@ extern "C" int nf_execute_sic_noalloc(const nf_sic *sic, void *stream) {
     const QueueClear qc{reinterpret_cast<int32_t *>(d + L.o_counter), nullptr, nullptr, 0};
     int e = launch_gather(pl, sl, true, nullptr, src, qc, st);
     if (!e)
-        e = launch_batched(reinterpret_cast<const SicView *>(d), s.cpd, s.softening, pc, TileShape{S, 64, 4, 0},
+        e = launch_batched(reinterpret_cast<const SicView *>(d), s.cpd, s.softening, pc, TileShape{S, 0, 0},
                            reinterpret_cast<const WorkItem *>(d + L.o_items), (int32_t)nitems, qc,
                            s.NSourceBlocks > 0, st);
     uint64_t r0, r1;
