@@ -1528,10 +1528,9 @@ __device__ __forceinline__ void tail_item(const BatchCtx &cx, const SicView &v, 
 }
 
 // Occupancy target WPE (waves per SIMD): more resident waves hide the v_rsq
-// and scalar-load latencies, as long as the tile loops' registers fit.  The
-// most waves at which each (pair form, sinks per lane) compiled with no VGPR
-// spills in its tile loops for gfx950 (6 waves: 80 VGPRs; 4: 128); S = 4 keeps
-// 4 waves, which measured faster than 5.
+// and scalar-load latencies, as long as the tile loops' registers fit (6 waves:
+// 80 VGPRs; 4: 128).  Only the cubic spline spills VGPRs, 4 of them at S = 1 and
+// 2; S = 4 keeps 4 waves, which measured faster than 5.
 constexpr int batched_waves_per_eu(int /*soft*/, int s) { return s == 4 ? 4 : 6; }
 
 }  // namespace
@@ -1647,7 +1646,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, 8))) v
 
 template <int S, int MODE, int WPE>
 int run_probe_t(const PairConst &pc, double *rate) {
-    constexpr int kSrc = 1024, kPasses = 2;  // ~0.3 s per launch at S = 2 on a full GPU
+    // 25 ms a launch at S = 2 on a full GPU: two passes, 0.4 ms, read 10-20% less
+    // than the loop's rate (4.35e12 interactions/s unsoftened at 6 waves).
+    constexpr int kSrc = 1024, kPasses = 128;
     int ncu = device_cu_count(), bpc = 0;
     if (ncu <= 0) return (int)hipErrorNoDevice;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_probe<NF_SOFT_SINGLE_SPLINE, S, MODE, WPE>,
