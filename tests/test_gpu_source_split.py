@@ -24,8 +24,8 @@ def _box(cpd, per_cell):
 
 # Pencils of no sinks, of one tail either side of the 43-sink line (a tail of 42
 # or a one-wave tile of 43 sinks), of whole tiles with and without a tail, and
-# of more than 64 source blocks; few enough cells that one SIC is below the
-# split's bound, and enough pairs in the heavy box that a group of SICs is not.
+# of more than 64 source blocks; few enough cells that a SIC is below the split's
+# bound.
 @pytest.mark.parametrize("per_cell", [(0, 0, 3), (8, 8, 9, 8, 9), (9, 8, 9), (13, 12), (64,), (27, 0, 0, 0), (900, 5)])
 @pytest.mark.parametrize("radius", [1, 2])
 def test_split_and_whole_tiles_bitwise(per_cell, radius):
